@@ -1,0 +1,127 @@
+"""The strict GEMM's fp16 products (csrc/nf24_gemm_f16.hip, calls of more than
+32 rows) where they can go wrong: tile edges, the row scale (outliers beyond
+its headroom, rows that begin with zeros, tiny and huge rows), infinities and
+NaNs, and codes over the format's whole range.
+
+Bound.  Each operand is carried as two fp16 values that hold it to one unit of
+fp32's last place, the dropped product of the low parts is below 2^-22 of the
+term, and the sums are fp32: within _parity.gemm_order_bound for K >= 64.  A
+value of x below 2^-24 of its row's scale is rounded to 2^-25 of the scale,
+2^-31 of the largest of the values the scale was set from (the row's first 32,
+or all of them when those are zero): 2^-31 * max|x_row| * sum_k |w_k| covers it.
+"""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from _parity import gemm_f64, gemm_order_bound, seeded_linear, stats
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(torch, x, c01, q2, s, b):
+    from tsplat.nf24 import nf24_linear
+
+    t = [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (x, c01, q2, s, b)]
+    return nf24_linear(*t).cpu().numpy()
+
+
+def _check(oracle, x, c01, q2, s, b, got):
+    w = oracle.decode_nf24(c01, q2, s)
+    floor = 2.0 ** -31 * np.abs(x.astype(np.float64)).max(1)[:, None] * np.abs(w.astype(np.float64)).sum(0)[None]
+    exact = gemm_f64(x, w, b)
+    assert np.all(np.isfinite(got))
+    assert np.all(np.abs(got - exact) <= gemm_order_bound(x, w, b) + floor), float(np.abs(got - exact).max())
+    return stats(got, exact)
+
+
+@pytest.mark.parametrize("M,K,N", [(33, 64, 4), (64, 1024, 1024), (127, 96, 68), (129, 100, 132), (255, 1024, 260),
+                                   (257, 68, 1028), (300, 1024, 3072), (511, 1056, 576), (2100, 1024, 1024),
+                                   (4100, 1000, 3072), (6500, 256, 2048), (8200, 64, 4096)])
+def test_tile_edges(oracle, cuda, hiplib, M, K, N):
+    import torch
+
+    print(f"gemm f16 M={M} K={K} N={N}", flush=True)
+    x, w, b = seeded_linear(M + K + N, M, K, N, w_scale=0.02)
+    c01, q2, s = oracle.quantize_nf24_i16(w)
+    got = _run(torch, x, c01, q2, s, b)
+    e = _check(oracle, x, c01, q2, s, b, got)
+    # against the sequential fp32 chain on some of the rows: no less exact
+    rows = np.random.default_rng(M).choice(M, min(M, 24), replace=False)
+    ref = oracle.nf24_gemm(x[rows], c01, q2, s, b)
+    exact = gemm_f64(x[rows], oracle.decode_nf24(c01, q2, s), b)
+    assert stats(got[rows], exact)["rmse"] <= 1.05 * stats(ref, exact)["rmse"] + 1e-12, e
+
+
+@pytest.mark.parametrize("M,N", [(40, 64), (300, 1024), (700, 576)])
+def test_row_scale(oracle, cuda, hiplib, M, N):
+    """Rows of every kind beside plain ones; the plain rows keep their bits."""
+    import torch
+
+    K = 160
+    x, w, b = seeded_linear(M + N, M, K, N, w_scale=0.02)
+    c01, q2, s = oracle.quantize_nf24_i16(w)
+    plain = _run(torch, x, c01, q2, s, b)
+    y = x.copy()
+    y[1, 40] = 3.0e5                      # beyond the headroom of the first 32 values
+    y[5, 159] = -7.0e9
+    y[9, :32] = 0.0                       # the scale comes from the rest
+    y[12, :] = 0.0
+    y[17] *= np.float32(1e-30)
+    y[21] *= np.float32(1e30)
+    y[25, :32] = 1e-20                    # the first values say nothing about the row
+    y[30] *= np.exp2(np.random.default_rng(3).integers(-20, 20, K)).astype(np.float32)
+    y[33, 0] = 1.0e6                      # large among the first 32
+    y[35, 100] = 3000.0                   # scaled, between fp16's largest value and twice that
+    changed = [1, 5, 9, 12, 17, 21, 25, 30, 33, 35]
+    got = _run(torch, y, c01, q2, s, b)
+    _check(oracle, y, c01, q2, s, b, got)
+    keep = np.setdiff1d(np.arange(M), changed)
+    assert np.array_equal(got[keep].view(np.uint32), plain[keep].view(np.uint32))
+    w64 = oracle.decode_nf24(c01, q2, s)
+    for r in (9, 17, 21, 25):             # rows of one magnitude: as exact as any other
+        zero = np.zeros_like(b)
+        one = _run(torch, y, c01, q2, s, zero)[r:r + 1]
+        assert stats(one, gemm_f64(y[r:r + 1], w64, zero))["rel_rmse"] < 1e-6
+
+
+@pytest.mark.parametrize("M,N", [(40, 64), (300, 1024)])
+def test_not_finite(oracle, cuda, hiplib, M, N):
+    """Infinities and NaNs of x give what the fp32 chain gives; other rows keep their bits."""
+    import torch
+
+    K = 96
+    x, w, b = seeded_linear(M + N + 1, M, K, N, w_scale=0.02)
+    c01, q2, s = oracle.quantize_nf24_i16(w)
+    c01[50, ::3], q2[50, ::3] = 0, 0      # inf * 0
+    plain = _run(torch, x, c01, q2, s, b)
+    y = x.copy()
+    y[2, 7] = np.inf
+    y[3, 50] = -np.inf
+    y[8, 95] = np.nan
+    y[11, [4, 60]] = np.inf, -np.inf
+    y[20, [3, 80]] = np.inf, 2.0e38
+    got = _run(torch, y, c01, q2, s, b)
+    ref = oracle.nf24_gemm(y, c01, q2, s, b)
+    bad = [2, 3, 8, 11, 20]
+    assert np.array_equal(np.isnan(got[bad]), np.isnan(ref[bad]))
+    inf = np.isinf(ref[bad])
+    assert np.array_equal(got[bad][inf], ref[bad][inf])
+    keep = np.setdiff1d(np.arange(M), bad)
+    assert np.array_equal(got[keep].view(np.uint32), plain[keep].view(np.uint32))
+
+
+def test_whole_code_range(oracle, cuda, hiplib):
+    """Any int16 / int8 code, not only the packer's."""
+    import torch
+
+    M, K, N = 64, 128, 64
+    r = np.random.default_rng(5)
+    c01 = r.integers(-32768, 32768, (K, N)).astype(np.int16)
+    q2 = r.integers(-128, 128, (K, N)).astype(np.int8)
+    c01[0, :4], q2[0, :4] = (32767, -32768, 32767, 0), (127, -128, -128, 1)
+    s = (r.random(N) * 1e-6).astype(np.float32)
+    x = r.standard_normal((M, K)).astype(np.float32)
+    b = r.standard_normal(N).astype(np.float32)
+    _check(oracle, x, c01, q2, s, b, _run(torch, x, c01, q2, s, b))

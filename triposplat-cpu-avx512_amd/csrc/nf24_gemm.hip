@@ -8,6 +8,11 @@
 // MFMA (v_mfma_f32_32x32x2_f32), so only the summation order differs from
 // the reference's sequential fmaf chain.
 //
+// Of the strict calls of more than 32 rows the fp16-product kernel
+// (nf24_gemm_f16.hip, 2.1-2.5x faster) takes all that its loads allow
+// (gemm_f16_takes); the tiles here serve the others, from 256 rows and
+// columns on.
+//
 // Tiling: a workgroup computes a BM x BN output tile with WM x WN waves; a
 // wave owns (BM/WM) x (BN/WN) = MB x NB blocks of 32x32.  Per K step of BK,
 // the X tile (fp32) and the decoded W tile (fp32) are staged in LDS, both
@@ -650,6 +655,8 @@ int launch_nf24_gemm(const GemmParams& p, hipStream_t stream) {
     if (p.M > 8 && p.K <= 256) return launch_cfg<CfgSkinny>(p, stream);
     return launch_nf24_gemv(p, stream);
   }
+  if (gemm_f16_takes(p))
+    return launch_gemm_f16(p, kEpiStore, QkvArgs{}, GemmEpilogueParams{kEpilogueStore, nullptr, 0, 1}, 0, stream);
   // The row tail goes first: its workspace is the only thing that can fail
   // (e.g. under graph capture), and then nothing has been enqueued.
   if (const int rem = tail_rows(p.M, p.n_count)) {
@@ -702,6 +709,7 @@ template <int kEpi>
 int launch_epi_kind(const GemmParams& p, const GemmEpilogueParams& e, hipStream_t stream,
                     const QkvArgs& q = QkvArgs{}, int row0 = 0) {
   if (p.precision != kPrecisionFp32 && p.M > 32) return launch_gemm_bf16(p, kEpi, q, e, row0, stream);
+  if (p.M > 32 && gemm_f16_takes(p)) return launch_gemm_f16(p, kEpi, q, e, row0, stream);
   // The row tail first (as in launch_nf24_gemm: only its workspace can fail).
   if (const int rem = tail_rows(p.M, p.n_count)) {
     const int st = launch_tail_rows<kEpi>(rows_slice(p, p.M - rem, rem), e, q, row0 + p.M - rem, stream);

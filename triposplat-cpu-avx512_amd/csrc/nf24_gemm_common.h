@@ -226,6 +226,9 @@ __device__ __forceinline__ void store_result(const GemmArgs& a, floatx16 (&acc)[
         const int col = col_base + nb * 32 + l32;
         const int rb = row_base + mb * 32;
         if (col >= a.n_count || rb >= a.M) continue;
+        // a block's addresses and gates are not computed beside another's
+        // (the 128-accumulator tiles would spill)
+        __builtin_amdgcn_sched_barrier(0);
         float* dst = a.out + (int64_t)rb * a.stride_out + col;
         float old[16], gt[16];
 #pragma unroll
@@ -301,6 +304,15 @@ inline bool vec_buffers_fit(const GemmParams& p, int bm, int bk) {
 // operands e, gate operands ep, token index of row 0 row0.
 int launch_gemm_bf16(const GemmParams& p, int epi, const QkvArgs& e, const GemmEpilogueParams& ep,
                      int row0, hipStream_t stream);
+
+// The strict GEMM of more than 32 rows on the fp16 matrix cores
+// (nf24_gemm_f16.hip), same arguments.  gemm_f16_takes: whether it serves the
+// call; gemm_f16_vector: whether the call's strides and alignment allow its
+// vector loads.
+bool gemm_f16_takes(const GemmParams& p);
+bool gemm_f16_vector(const GemmParams& p);
+int launch_gemm_f16(const GemmParams& p, int epi, const QkvArgs& e, const GemmEpilogueParams& ep,
+                    int row0, hipStream_t stream);
 
 // A row tail (at most 32 rows, token index of its row 0 row0) split off a
 // bf16-mode call, on the strict few-row path (nf24_gemm.hip) with epilogue
