@@ -108,9 +108,10 @@ int triposplat_sdpa_f32_avx512_exact_q8t512_packed_blhd(
  * and query block report this library's tiles (64 keys, 128 queries).
  * Profile: calls and wall time of the blocking calls (allocate/pack/free
  * report 0: there is no per-call workspace or pack step).
- * Workspace: the SDPA's key-split partials, and the bf16 modes' pre-split
- * K/V image, live in grow-only device buffers, one per (device, stream, use);
- * stats report their allocations and bytes together.
+ * Workspace: the SDPA's key-split partials, and the pre-split K/V image of
+ * the strict kernel (with the partials, 512 bytes per key and head) and of
+ * the bf16 modes, live in grow-only device buffers, one per (device, stream,
+ * use); stats report their allocations and bytes together.
  * Release frees, after its stream, the buffer of every stream on the current
  * device that is idle, and keeps (until the process ends) the buffers a HIP
  * graph captured, those of a stream under capture at that moment (waiting on

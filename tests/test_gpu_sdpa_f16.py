@@ -1,0 +1,130 @@
+"""The strict SDPA's fp16 products (csrc/sdpa_f16.hip, from 64 keys on) where
+they can go wrong: ragged tiles around the key tile and both workgroup sizes,
+the scales of q, k and v, references that move, huge scores and masks, and
+infinities.  Against the float64 formula; the fp32 oracle's own error is the
+yardstick where the inputs are plain."""
+from __future__ import annotations
+
+import math
+
+import numpy as np
+import pytest
+
+from _parity import sdpa_f64, stats
+from test_gpu_sdpa import _qkv, _run
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("H,Lq,Lk,bias", [(2, 1, 64, None), (2, 33, 65, "one"), (3, 129, 127, None),
+                                          (1, 128, 1023, "uniform"), (2, 65, 1025, None), (1, 31, 2111, "one"),
+                                          (16, 8200, 130, "uniform"), (16, 4100, 1090, None)])
+def test_sizes(oracle, cuda, H, Lq, Lk, bias, packed):
+    import torch
+
+    print(f"sdpa f16 H={H} Lq={Lq} Lk={Lk} bias={bias} packed={packed}", flush=True)
+    q, k, v = _qkv(Lq + Lk, 1, H, Lq, Lk)
+    b = None
+    if bias == "one":
+        b = np.zeros(Lk, np.float32)
+        b[Lk - 1] = math.log(Lk)
+    elif bias == "uniform":
+        b = np.random.default_rng(3).uniform(-2, 0, Lk).astype(np.float32)
+    got = _run(torch, cuda, q, k, v, b, packed=packed)
+    rows = np.unique(np.r_[0:min(Lq, 24), max(0, Lq - 24):Lq])
+    exact = sdpa_f64(q[:, :, rows], k, v, b)
+    ref = oracle.sdpa_q8t512(np.ascontiguousarray(q[:, :, rows]), k, v, b)
+    got = got[:, :, rows]
+    assert np.all(np.isfinite(got))
+    assert stats(got, exact)["rmse"] <= 1.1 * stats(ref, exact)["rmse"] + 2.0 ** -24 * float(np.abs(v).max())
+
+
+@pytest.mark.parametrize("Lk", [200, 1100])
+def test_scales(cuda, Lk):
+    """q rows, heads of k and of v at any magnitude; tokens far below their head's largest."""
+    import torch
+
+    q, k, v = _qkv(9, 1, 4, 70, Lk)
+    plain = _run(torch, cuda, q, k, v)
+    # powers of two that cancel in the scores change no bit
+    q2, k2 = q.copy(), k.copy()
+    q2[:, 1] *= np.float32(2.0 ** -40)
+    k2[:, 1] *= np.float32(2.0 ** 40)
+    q2[:, 2] *= np.float32(2.0 ** 30)
+    k2[:, 2] *= np.float32(2.0 ** -30)
+    assert np.array_equal(_run(torch, cuda, q2, k2, v).view(np.uint32), plain.view(np.uint32))
+    v2 = v * np.float32(2.0 ** -60)
+    assert np.array_equal(_run(torch, cuda, q, k, v2) * np.float32(2.0 ** 60), plain)
+    k2, v2 = k.copy(), v.copy()
+    k2[:, :, 5::7] *= np.float32(1e-4)
+    v2[:, :, 3::5] *= np.float32(1e3)
+    got, exact = _run(torch, cuda, q, k2, v2), sdpa_f64(q, k2, v2)
+    assert stats(got, exact)["rel_rmse"] < 2e-6
+    z = np.zeros_like(k)
+    assert stats(_run(torch, cuda, q, z, v), sdpa_f64(q, z, v))["rel_rmse"] < 1e-6
+    assert np.all(_run(torch, cuda, q, k, np.zeros_like(v)) == 0)
+
+
+@pytest.mark.parametrize("scale", [30.0, 1e3, 1e5, 1e7])
+def test_huge_scores(cuda, scale):
+    """One key holds all the weight: its value, whatever the scores' size."""
+    import torch
+
+    q, k, v = _qkv(11, 1, 2, 70, 300)
+    q, k = (q * np.float32(scale)).astype(np.float32), (k * np.float32(scale)).astype(np.float32)
+    top = np.argsort(np.einsum("bhqd,bhkd->bhqk", q.astype(np.float64), k.astype(np.float64)), -1)
+    got = _run(torch, cuda, q, k, v)
+    exact = sdpa_f64(q, k, v)
+    assert np.all(np.isfinite(got)) and top.shape[-1] == 300
+    assert stats(got, exact)["rel_rmse"] < (1e-4 if scale < 100 else 1e-6)
+
+
+@pytest.mark.parametrize("value", [-1e4, -1e8, -1e30])
+@pytest.mark.parametrize("Lq", [70, 8200])
+def test_masks(oracle, cuda, value, Lq):
+    """Additive masks over leading, trailing and all keys, on both workgroup sizes."""
+    import torch
+
+    H, Lk = (2, 300) if Lq < 100 else (16, 300)
+    q, k, v = _qkv(13, 1, H, Lq, Lk)
+    rows = np.arange(0, 70)
+    for cols in (slice(0, 100), slice(100, 300), slice(0, 299), slice(0, 300)):
+        b = np.zeros(Lk, np.float32)
+        b[cols] = value
+        got = _run(torch, cuda, q, k, v, b)
+        assert np.all(np.isfinite(got))
+        if cols != slice(0, 300) or value != -1e8:  # (there fp32 holds the scores to 8)
+            exact = sdpa_f64(q[:, :, rows], k, v, b)
+            assert stats(got[:, :, rows], exact)["max_abs"] < (2e-3 if cols == slice(0, 300) and value == -1e4 else 1e-5)
+
+
+def test_not_finite(cuda):
+    """An infinite k makes the scores it should (no weight, or NaN); an infinite
+    or NaN v reaches the outputs of its dim and no others; a NaN q its row."""
+    import torch
+
+    q, k, v = _qkv(15, 1, 2, 66, 130)
+    base = _run(torch, cuda, q, k, v)
+    v2 = v.copy()
+    v2[0, 0, 100, 7] = np.inf
+    v2[0, 0, 3, 9] = np.nan
+    got = _run(torch, cuda, q, k, v2)
+    assert np.all(got[0, 0, :, 7] == np.inf) and np.all(np.isnan(got[0, 0, :, 9]))
+    keep = np.setdiff1d(np.arange(64), [7, 9])
+    assert np.array_equal(got[0, 0][:, keep], base[0, 0][:, keep]) and np.array_equal(got[0, 1], base[0, 1])
+    k2 = k.copy()
+    k2[0, 1, 77, 5] = -np.inf
+    got = _run(torch, cuda, q, k2, v)
+    drop = np.setdiff1d(np.arange(130), [77])
+    exact = sdpa_f64(q, k[:, :, drop], v[:, :, drop])
+    up = q[0, 1, :, 5] > 0                                  # score -inf: the key has no weight
+    assert stats(got[0, 1][up], exact[0, 1][up])["max_abs"] < 1e-5
+    assert np.all(np.isnan(got[0, 1][~up]))                 # score +inf
+    assert np.array_equal(got[0, 0], base[0, 0])
+    q2 = q.copy()
+    q2[0, 0, 4, 60] = np.nan
+    got = _run(torch, cuda, q2, k, v)
+    assert np.all(np.isnan(got[0, 0, 4]))
+    rest = np.setdiff1d(np.arange(66), [4])
+    assert np.array_equal(got[0, 0][rest], base[0, 0][rest])

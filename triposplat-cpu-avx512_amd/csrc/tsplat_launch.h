@@ -77,6 +77,8 @@ void note_sdpa_query_tile(int queries);
 int sdpa_query_tile();
 // The bf16-MFMA modes (called by launch_sdpa for precision != fp32).
 int launch_sdpa_bf16(const SdpaParams& p, hipStream_t stream);
+// The strict SDPA on the fp16 matrix cores (called by launch_sdpa).
+int launch_sdpa_f16(const SdpaParams& p, hipStream_t stream);
 
 // qkv [B*L, 3*H*64] -> RoPE then RMSNorm on q and k; q [B, H, L, 64],
 // packed k/v [B, H, 64, L_padded] with tokens L..L_padded-1 zero.
