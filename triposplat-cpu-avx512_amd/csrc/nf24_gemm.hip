@@ -9,7 +9,7 @@
 // the reference's sequential fmaf chain.
 //
 // Of the strict calls of more than 32 rows the fp16-product kernel
-// (nf24_gemm_f16.hip, 2.1-2.5x faster) takes all that its loads allow
+// (nf24_gemm_f16.hip, 2.1-2.7x faster) takes all that its loads allow
 // (gemm_f16_takes); the tiles here serve the others, from 256 rows and
 // columns on.
 //

@@ -41,14 +41,21 @@
 // swizzled as in nf24_gemm_bf16.hip: chunk c of row r sits at position
 // c ^ ((r >> 2) & 3) and W tile column r in LDS row w_row(r), which keeps
 // the 128-bit fragment reads and the staging stores off each other's banks.
-// LDS is double-buffered with one barrier per step; the next step's x and
-// codes are fetched into registers while the current step's MFMAs run.
+// LDS is double-buffered with one barrier per step.  A step's MFMAs run in
+// groups of 3 * kNB, and each group carries a share of the next step's staging
+// between them: a unit is split or decoded and stored from registers that were
+// loaded a step earlier, and the step after that is loaded into them, so no
+// wave waits for memory inside a step.  (Staged after the MFMAs instead, from
+// loads of the same step: 4096 x 1024 x 3072 84 us, 12294 x 4096 x 1024 350,
+// fused QKV over 8194 rows 261, 600 x 1024 x 1024 34.)
 //
-// Measured against the fp32 MFMA tiles: 4096 x 1024 x 3072 197 -> 85 us (305
-// TFLOP/s), 12294 x 4096 x 1024 788 -> 328 us, 12294 x 1024 x 4096 765 -> 310
-// us, 600 x 1024 x 1024 47 -> 34 us.  What bounds it: a K step of the 256 x
-// 256 tile is 3072 cycles of MFMA and about 2000 of staging (the splits, the
-// decode, the LDS stores and the barrier), which follow one another.
+// Measured against the fp32 MFMA tiles: 4096 x 1024 x 3072 197 -> 78 us (330
+// TFLOP/s), 12294 x 4096 x 1024 788 -> 284 us (363), 12294 x 1024 x 4096 765 ->
+// 299 us, fused QKV over 8194 rows 496 -> 233 us, 600 x 1024 x 1024 47 -> 32
+// us.  What bounds it: the fp16 matrix cores at the clock they hold; three
+// products at 363 TFLOP/s are 1.09 PFLOP/s, a plain 8192^3 fp16 library product
+// on the same card 1.11.  Grids of one round or less are bound by a tile's
+// chain of K steps instead (31 us at K = 1024 for the smallest).
 
 #include "nf24_gemm_common.h"
 
@@ -90,9 +97,7 @@ struct F16Cfg {
 
 __device__ __forceinline__ int chunk_offset(int r, int c) { return r * 32 + ((c ^ ((r >> 2) & 3)) << 3); }
 __device__ __forceinline__ int w_row(int r) { return r ^ (((r >> 4) & 1) | ((r >> 5) & 2)); }
-__device__ __forceinline__ half8 lds_frag(const _Float16* base, int r, int c) {
-  return *reinterpret_cast<const half8*>(base + chunk_offset(r, c));
-}
+__device__ __forceinline__ half8 lds_frag(const _Float16* src) { return *reinterpret_cast<const half8*>(src); }
 __device__ __forceinline__ floatx16 mfma_f16(const half8& a, const half8& b, floatx16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
 }
@@ -106,11 +111,13 @@ __device__ __forceinline__ void split2(float a, float b, float hi_a, float hi_b,
 }
 
 // p / 256 of column e of a staged unit row (two int16 codes per word, four
-// int8 codes per word): exact in fp32.
-__device__ __forceinline__ float w_payload(const uint32_t (&c)[2], uint32_t q, int e) {
-  const int32_t code = (int32_t)(int16_t)(c[e >> 1] >> (16 * (e & 1)));
-  const int32_t q2 = (int32_t)(int8_t)(q >> (8 * e));
-  return (float)(code * 256 + q2) * 0.00390625f;
+// int8 codes per word, these with their sign bits flipped): the bytes side by
+// side are (p + 128) * 256 as an int32, of at most 24 significant bits, so
+// the conversion and the difference are exact in fp32.
+constexpr uint32_t kFlipQ2 = 0x80808080u;
+__device__ __forceinline__ float w_payload(const uint32_t (&c)[2], uint32_t q_flipped, int e) {
+  const uint32_t sel = ((e & 1) ? 0x0706000cu : 0x0504000cu) | ((uint32_t)e << 8);
+  return fmaf((float)(int32_t)__builtin_amdgcn_perm(c[e >> 1], q_flipped, sel), 0x1p-16f, -0.5f);
 }
 
 template <int NW>
@@ -127,6 +134,14 @@ __device__ __forceinline__ float row_scale(uint32_t mx_bits) {
 }
 __device__ __forceinline__ float inverse_pow2(float s) {
   return __uint_as_float((254u << 23) - __float_as_uint(s));
+}
+
+// Largest of x over eight lanes (a swizzle has no lane addresses to hold, and
+// so none that the QKV epilogue would share and keep over the K loop).
+__device__ __forceinline__ uint32_t max8(uint32_t x) {
+  x = max(x, (uint32_t)__builtin_amdgcn_ds_swizzle((int)x, (1 << 10) | 0x1f));  // lane ^ 1
+  x = max(x, (uint32_t)__builtin_amdgcn_ds_swizzle((int)x, (2 << 10) | 0x1f));
+  return max(x, (uint32_t)__builtin_amdgcn_ds_swizzle((int)x, (4 << 10) | 0x1f));
 }
 
 // kVec: x rows 16-byte aligned with K % 4 == 0; N, n_start, n_count
@@ -174,8 +189,11 @@ void nf24_gemm_f16_kernel(GemmArgs a) {
   uint32_t cr[C::kWIter][C::WK][2];    // k row i: int16 codes of columns 0,1 | 2,3
   uint32_t qr[C::kWIter][C::WK];       // k row i: int8 codes of columns 0..3
 
+  // code element offset past both planes: itself and doubled (mod 2^32) it is
+  // at least kBufOob, whatever in-range step is added
+  constexpr uint32_t kWOob = 0xc0000000u;
   __amdgpu_buffer_rsrc_t rx, rc, rq;
-  uint32_t x_off[C::kXIter], c_off[C::kWIter], q_off[C::kWIter];
+  uint32_t x_off[C::kXIter], w_off[C::kWIter];
   if constexpr (kVec) {
     rx = buffer_rsrc(a.x + (int64_t)m0 * a.stride_x, ((int64_t)(rows - 1) * a.stride_x + a.K) * 4);
 #pragma unroll
@@ -189,8 +207,7 @@ void nf24_gemm_f16_kernel(GemmArgs a) {
 #pragma unroll
     for (int j = 0; j < C::kWIter; ++j) {
       const uint32_t e = (uint32_t)(w_k[j] * a.N + a.n_start + c0 + w_col[j]);
-      c_off[j] = w_ok[j][0] ? 2u * e : kBufOob;
-      q_off[j] = w_ok[j][0] ? e : kBufOob;
+      w_off[j] = w_ok[j][0] ? e : kWOob;
     }
   }
 
@@ -213,74 +230,85 @@ void nf24_gemm_f16_kernel(GemmArgs a) {
     }
     return v;
   };
+  // W unit j (WK code rows of 4 columns) of the step at k0.
+  auto load_w = [&](int j, int k0) {
+#pragma unroll
+    for (int i = 0; i < C::WK; ++i) {
+      if constexpr (kVec) {
+        const uint32_t e = w_off[j] + (uint32_t)(k0 + i) * (uint32_t)a.N;
+        const auto c = __builtin_amdgcn_raw_buffer_load_b64(rc, (int)(2u * e), 0, 0);
+        cr[j][i][0] = c[0];
+        cr[j][i][1] = c[1];
+        qr[j][i] = __builtin_amdgcn_raw_buffer_load_b32(rq, (int)e, 0, 0);
+      } else {
+        const int gk = k0 + w_k[j] + i;
+        const int64_t off = (int64_t)gk * a.N + a.n_start + c0 + w_col[j];
+        uint32_t c[4], q = 0u;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const bool ok = w_ok[j][e] && gk < a.K;
+          c[e] = ok ? (uint16_t)a.code01[off + e] : 0u;
+          q |= (ok ? (uint32_t)(uint8_t)a.q2[off + e] : 0u) << (8 * e);
+        }
+        cr[j][i][0] = c[0] | (c[1] << 16);
+        cr[j][i][1] = c[2] | (c[3] << 16);
+        qr[j][i] = q;
+      }
+    }
+  };
   auto load_tile = [&](int k0) {
 #pragma unroll
     for (int j = 0; j < C::kXIter; ++j)
       if (x_unit(j)) xr[j] = load_x(j, k0);
 #pragma unroll
-    for (int j = 0; j < C::kWIter; ++j) {
-      if (!w_unit(j)) continue;
-#pragma unroll
-      for (int i = 0; i < C::WK; ++i) {
-        if constexpr (kVec) {
-          const uint32_t e = (uint32_t)(k0 + i) * (uint32_t)a.N;
-          const auto c = __builtin_amdgcn_raw_buffer_load_b64(rc, (int)(c_off[j] + 2u * e), 0, 0);
-          cr[j][i][0] = c[0];
-          cr[j][i][1] = c[1];
-          qr[j][i] = __builtin_amdgcn_raw_buffer_load_b32(rq, (int)(q_off[j] + e), 0, 0);
-        } else {
-          const int gk = k0 + w_k[j] + i;
-          const int64_t off = (int64_t)gk * a.N + a.n_start + c0 + w_col[j];
-          uint32_t c[4], q = 0u;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const bool ok = w_ok[j][e] && gk < a.K;
-            c[e] = ok ? (uint16_t)a.code01[off + e] : 0u;
-            q |= (ok ? (uint32_t)(uint8_t)a.q2[off + e] : 0u) << (8 * e);
-          }
-          cr[j][i][0] = c[0] | (c[1] << 16);
-          cr[j][i][1] = c[2] | (c[3] << 16);
-          qr[j][i] = q;
-        }
-      }
-    }
+    for (int j = 0; j < C::kWIter; ++j)
+      if (w_unit(j)) load_w(j, k0);
   };
 
-  // limit: bound of xh, infinite in the first pass
-  auto store_tile = [&](int buf, float limit) {
+  // A step's staging in kStages parts: x unit j, then column e of W unit j.
+  // A part places its values in LDS buffer buf and, its registers free, loads
+  // the step at k_next into them.  limit: bound of xh, infinite in the first
+  // pass.
+  // LDS positions: x units of a thread are a multiple of 16 rows apart, and
+  // the four columns of a W unit (w_col a multiple of 4) are rows whose two
+  // low bits alone differ.
+  static_assert(C::kThreads / (C::BK / 4) % 16 == 0, "x units keep the swizzle");
+  // 4-k unit kc of a row: chunk kc/2, half kc%2
+  const int x_dst = chunk_offset(tid / (C::BK / 4), (tid % (C::BK / 4)) >> 1) + 4 * (tid & 1);
+  int w_dst[C::kWIter];
 #pragma unroll
-    for (int j = 0; j < C::kXIter; ++j) {
-      if (!x_unit(j)) continue;
-      const int idx = tid + j * C::kThreads;
-      const int row = idx / (C::BK / 4);
-      const int kc = idx % (C::BK / 4);  // 4-k unit: chunk kc/2, half kc%2
-      const floatx4 v = xr[j] * row_sc[row];
+  for (int j = 0; j < C::kWIter; ++j) w_dst[j] = chunk_offset(w_row(w_col[j]), w_k[j] >> 3) + (w_k[j] & 7);
+  constexpr int kStages = C::kXIter + 4 * C::kWIter;
+  float rsc[C::kXIter];  // scale of x unit j's row
+  auto stage = [&](int part, int buf, float limit, int k_next) {
+    if (part < C::kXIter) {
+      const int j = part;
+      if (!x_unit(j)) return;
+      const floatx4 v = xr[j] * rsc[j];
       float m[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) m[e] = __builtin_amdgcn_fmed3f(v[e], -limit, limit);
       unsigned hi[2], lo[2];
       split2(v[0], v[1], m[0], m[1], hi[0], lo[0]);
       split2(v[2], v[3], m[2], m[3], hi[1], lo[1]);
-      const int off = chunk_offset(row, kc >> 1) + 4 * (kc & 1);
+      const int off = x_dst + j * (C::kThreads / (C::BK / 4)) * 32;
       store_pairs(&xs[buf][0][off], hi);
       store_pairs(&xs[buf][1][off], lo);
-    }
+      xr[j] = load_x(j, k_next);
+    } else {
+      const int j = (part - C::kXIter) / 4, e = (part - C::kXIter) % 4;
+      if (!w_unit(j)) return;
+      unsigned hi[C::WK / 2], lo[C::WK / 2];
 #pragma unroll
-    for (int j = 0; j < C::kWIter; ++j) {
-      if (!w_unit(j)) continue;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        unsigned hi[C::WK / 2], lo[C::WK / 2];
-#pragma unroll
-        for (int i = 0; i < C::WK / 2; ++i) {
-          const float p0 = w_payload(cr[j][2 * i], qr[j][2 * i], e);
-          const float p1 = w_payload(cr[j][2 * i + 1], qr[j][2 * i + 1], e);
-          split2(p0, p1, p0, p1, hi[i], lo[i]);
-        }
-        const int off = chunk_offset(w_row(w_col[j] + e), w_k[j] >> 3) + (w_k[j] & 7);
-        store_pairs(&ws[buf][0][off], hi);
-        store_pairs(&ws[buf][1][off], lo);
+      for (int i = 0; i < C::WK / 2; ++i) {
+        const float p0 = w_payload(cr[j][2 * i], qr[j][2 * i] ^ kFlipQ2, e);
+        const float p1 = w_payload(cr[j][2 * i + 1], qr[j][2 * i + 1] ^ kFlipQ2, e);
+        split2(p0, p1, p0, p1, hi[i], lo[i]);
       }
+      const int off = w_dst[j] ^ (e * 32);
+      store_pairs(&ws[buf][0][off], hi);
+      store_pairs(&ws[buf][1][off], lo);
+      if (e == 3) load_w(j, k_next);
     }
   };
 
@@ -295,18 +323,23 @@ void nf24_gemm_f16_kernel(GemmArgs a) {
 #pragma unroll
       for (int e = 0; e < 4; ++e)
         if (k + 4 * (idx % (C::BK / 4)) + e < a.K) mx = max(mx, __float_as_uint(src[k + e]) & 0x7fffffffu);
-#pragma unroll
-    for (int d = 1; d < 8; d <<= 1) mx = max(mx, (uint32_t)__shfl_xor((int)mx, d));
+    mx = max8(mx);
     return mx;
   };
   auto set_scale = [&](int idx, uint32_t mx) {
     if (idx < C::kXUnits && idx % (C::BK / 4) == 0) row_sc[idx / (C::BK / 4)] = row_scale(mx);
   };
 
+  // vector ALU instructions between two MFMAs of a step: the staging's share
+  constexpr int kStageAlu = 5;
   floatx16 acc[C::kMB][C::kNB];
   const int nk = (a.K + C::BK - 1) / C::BK;
-  const int arow = wm * C::kTM + l32;
-  const int bcol = wn * C::kTN + l32;
+  // Fragment positions: a step of 32 rows or columns moves neither the
+  // swizzle nor (kTN = 32 * kNB, kNB <= 2) what w_row adds, 16 k flip bit 1 of
+  // the chunk.
+  static_assert(C::kNB <= 2, "w_row over the wave's columns");
+  const int a_src = chunk_offset(wm * C::kTM + l32, g);
+  const int b_src = chunk_offset(w_row(wn * C::kTN + l32), g);
 
   load_tile(0);
 #pragma unroll
@@ -316,8 +349,7 @@ void nf24_gemm_f16_kernel(GemmArgs a) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) mx = max(mx, __float_as_uint(xr[j][e]) & 0x7fffffffu);
     }
-#pragma unroll
-    for (int d = 1; d < 8; d <<= 1) mx = max(mx, (uint32_t)__shfl_xor((int)mx, d));
+    mx = max8(mx);
     // rows whose first 32 values are zero: the rest of the row decides
     const int idx = tid + j * C::kThreads;
     const bool zero = mx == 0 && x_unit(j) && idx / (C::BK / 4) < rows;
@@ -331,9 +363,68 @@ void nf24_gemm_f16_kernel(GemmArgs a) {
   // the code for both passes, the second being the exception.
   if (tid == 0) second = 0;
   __syncthreads();
+  // One K step on LDS buffer P: 2 * kMB groups of MFMAs (16 k, one row block),
+  // each with the fragment reads of the next group and, in all but the last
+  // step, a share of the next step's staging between its MFMAs.
+  auto step = [&](auto staged, int P, float limit, int k_next) {
+    constexpr int kGroups = 2 * C::kMB;
+    half8 ah[2], al[2], bh[2][C::kNB], bl[2][C::kNB];
+    auto read_a = [&](int grp) {
+      const int off = (a_src ^ (grp / C::kMB * 16)) + grp % C::kMB * 32 * 32;
+      ah[grp & 1] = lds_frag(&xs[P][0][off]);
+      al[grp & 1] = lds_frag(&xs[P][1][off]);
+    };
+    auto read_b = [&](int s) {
+#pragma unroll
+      for (int nb = 0; nb < C::kNB; ++nb) {
+        const int off = (b_src ^ (s * 16)) + nb * 32 * 32;
+        bh[s][nb] = lds_frag(&ws[P][0][off]);
+        bl[s][nb] = lds_frag(&ws[P][1][off]);
+      }
+    };
+    // two waves a SIMD have the registers to read a group ahead; the shapes
+    // of three and more have another wave to run while they wait
+    constexpr bool kAhead = C::kMinWaves <= 2;
+    if (kAhead) {
+      read_b(0);
+      read_a(0);
+    }
+#pragma unroll
+    for (int grp = 0; grp < kGroups; ++grp) {
+      const int s = grp / C::kMB, mb = grp % C::kMB;
+      if (!kAhead) {
+        if (mb == 0) read_b(s);
+        read_a(grp);
+      } else if (grp + 1 < kGroups) {
+        if (mb + 1 == C::kMB) read_b(s + 1);
+        read_a(grp + 1);
+      }
+#pragma unroll
+      for (int nb = 0; nb < C::kNB; ++nb) acc[mb][nb] = mfma_f16(ah[grp & 1], bh[s][nb], acc[mb][nb]);
+#pragma unroll
+      for (int nb = 0; nb < C::kNB; ++nb) acc[mb][nb] = mfma_f16(ah[grp & 1], bl[s][nb], acc[mb][nb]);
+#pragma unroll
+      for (int nb = 0; nb < C::kNB; ++nb) acc[mb][nb] = mfma_f16(al[grp & 1], bh[s][nb], acc[mb][nb]);
+      if constexpr (decltype(staged)::value) {
+#pragma unroll
+        for (int u = grp * kStages / kGroups; u < (grp + 1) * kStages / kGroups; ++u)
+          stage(u, P ^ 1, limit, k_next);
+        // an MFMA, then what fits beside it (mask 8: MFMA, 2: vector ALU)
+#pragma unroll
+        for (int i = 0; i < 3 * C::kNB; ++i) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x002, kStageAlu, 0);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
   for (;;) {
     const float limit = __builtin_amdgcn_readfirstlane(second) != 0 ? 65504.0f : INFINITY;
-    store_tile(0, limit);
+#pragma unroll
+    for (int j = 0; j < C::kXIter; ++j) rsc[j] = row_sc[x_unit(j) ? (tid + j * C::kThreads) / (C::BK / 4) : 0];
+#pragma unroll
+    for (int u = 0; u < kStages; ++u) stage(u, 0, limit, min(1, nk - 1) * C::BK);
     __syncthreads();
 #pragma unroll
     for (int mb = 0; mb < C::kMB; ++mb)
@@ -341,37 +432,13 @@ void nf24_gemm_f16_kernel(GemmArgs a) {
       for (int nb = 0; nb < C::kNB; ++nb)
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[mb][nb][r] = 0.0f;
-    for (int kt = 0; kt < nk; ++kt) {
-      const int P = kt & 1;
-      if (kt + 1 < nk) load_tile((kt + 1) * C::BK);
-#pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        const int ch = 2 * s + g;
-        half8 ah[C::kMB], bh[C::kNB], al[C::kMB], bl[C::kNB];
-#pragma unroll
-        for (int mb = 0; mb < C::kMB; ++mb) ah[mb] = lds_frag(xs[P][0], arow + mb * 32, ch);
-#pragma unroll
-        for (int nb = 0; nb < C::kNB; ++nb) bh[nb] = lds_frag(ws[P][0], w_row(bcol + nb * 32), ch);
-#pragma unroll
-        for (int mb = 0; mb < C::kMB; ++mb)
-#pragma unroll
-          for (int nb = 0; nb < C::kNB; ++nb) acc[mb][nb] = mfma_f16(ah[mb], bh[nb], acc[mb][nb]);
-#pragma unroll
-        for (int nb = 0; nb < C::kNB; ++nb) bl[nb] = lds_frag(ws[P][1], w_row(bcol + nb * 32), ch);
-#pragma unroll
-        for (int mb = 0; mb < C::kMB; ++mb)
-#pragma unroll
-          for (int nb = 0; nb < C::kNB; ++nb) acc[mb][nb] = mfma_f16(ah[mb], bl[nb], acc[mb][nb]);
-#pragma unroll
-        for (int mb = 0; mb < C::kMB; ++mb) al[mb] = lds_frag(xs[P][1], arow + mb * 32, ch);
-#pragma unroll
-        for (int mb = 0; mb < C::kMB; ++mb)
-#pragma unroll
-          for (int nb = 0; nb < C::kNB; ++nb) acc[mb][nb] = mfma_f16(al[mb], bh[nb], acc[mb][nb]);
-      }
-      if (kt + 1 < nk) store_tile(P ^ 1, limit);
+    for (int kt = 0; kt + 1 < nk; ++kt) {
+      // (the last staged step loads its own tile again, unused)
+      step(std::true_type{}, kt & 1, limit, min(kt + 2, nk - 1) * C::BK);
       __syncthreads();
     }
+    step(std::false_type{}, (nk - 1) & 1, limit, 0);
+    __syncthreads();
     // 0 * acc is NaN for an accumulator that is not finite
     float chk = 0.0f;
 #pragma unroll
@@ -483,14 +550,14 @@ int launch_cfg(const GemmArgs& a, int epi, hipStream_t stream) {
 
 // The tile shapes the launch model chooses from: a round of the chip
 // (CUs x wgs_per_cu workgroups) costs `round` us at K = 1024, measured on
-// grids of one to four rounds; the model is rounds x cost, a partial round as
-// much as a whole one (one workgroup alone takes 80 us of the 256 x 256
-// tile's 113: its K steps are a chain of staging and MFMA phases).
+// grids of one to twelve full rounds; the model is rounds x cost, a partial
+// round as much as a whole one (a nearly empty one takes 70, 56, 56, 42 and 31
+// us: its K steps follow one another at any load).
 struct F16Choice {
   int bm, bn, wgs_per_cu, round;
 };
 constexpr F16Choice kChoices[] = {
-    {256, 256, 1, 113}, {256, 192, 1, 89}, {192, 256, 1, 90}, {256, 128, 1, 60}, {128, 64, 2, 40}};
+    {256, 256, 1, 94}, {256, 192, 1, 82}, {192, 256, 1, 75}, {256, 128, 1, 57}, {128, 64, 2, 38}};
 constexpr int kNumChoices = sizeof(kChoices) / sizeof(kChoices[0]);
 
 int64_t model_time(int i, int M, int n_count) {
