@@ -278,6 +278,17 @@ int tsplat_nf24_pack_async(const float* weight, int out_features, int in_feature
                            const float* alphabet, int alphabet_len, float* base_workspace,
                            int16_t* code01_t, int8_t* q2_t, float* scale, void* stream);
 
+/* The same with the packer's error figures, reduced in the packing pass:
+ * stats is 8-byte aligned device memory of tsplat_nf24_pack_stats_bytes
+ * (out_features, in_features) bytes, or null; its first 9 doubles receive the
+ * sums of squares of the residuals after q0, q1, q2 and of the weights, the
+ * three residuals' largest magnitudes, and how many q1 and q2 were clamped. */
+int64_t tsplat_nf24_pack_stats_bytes(int out_features, int in_features);
+int tsplat_nf24_pack_stats_async(const float* weight, int out_features, int in_features,
+                                 const float* alphabet, int alphabet_len, float* base_workspace,
+                                 int16_t* code01_t, int8_t* q2_t, float* scale, double* stats,
+                                 void* stream);
+
 /* scripts/native_linear_nf24_prepacked.py:17-36 (decode_nf24_i16_weight_t /
  * decode_nf24_i16_weight): exact fp32 weights, out [in, out] like the codes,
  * or [out, in] (the nn.Linear layout) when transposed != 0. */

@@ -592,9 +592,21 @@ int tsplat_nf24_bf16_planes_async(const int16_t* code01_t, const int8_t* q2_t, c
 }
 
 // ------------------------------------------------------------------ packer
+int64_t tsplat_nf24_pack_stats_bytes(int out_features, int in_features) {
+  return out_features <= 0 || in_features <= 0 ? 0 : nf24_pack_stats_bytes(out_features, in_features);
+}
+
 int tsplat_nf24_pack_async(const float* weight, int out_features, int in_features,
                            const float* alphabet, int alphabet_len, float* base_workspace,
                            int16_t* code01_t, int8_t* q2_t, float* scale, void* stream) {
+  return tsplat_nf24_pack_stats_async(weight, out_features, in_features, alphabet, alphabet_len,
+                                      base_workspace, code01_t, q2_t, scale, nullptr, stream);
+}
+
+int tsplat_nf24_pack_stats_async(const float* weight, int out_features, int in_features,
+                                 const float* alphabet, int alphabet_len, float* base_workspace,
+                                 int16_t* code01_t, int8_t* q2_t, float* scale, double* stats,
+                                 void* stream) {
   if (!weight || !alphabet || !base_workspace || !code01_t || !q2_t || !scale) return kErrNull;
   if (out_features <= 0 || in_features <= 0 || alphabet_len < 2 || alphabet_len > 256)
     return kErrDims;
@@ -606,8 +618,12 @@ int tsplat_nf24_pack_async(const float* weight, int out_features, int in_feature
   TSPLAT_CHECK(ptrs.check(code01_t, count * 2));
   TSPLAT_CHECK(ptrs.check(q2_t, count));
   TSPLAT_CHECK(ptrs.check(scale, (int64_t)out_features * 4));
+  if (stats != nullptr) {
+    if (reinterpret_cast<uintptr_t>(stats) % alignof(double) != 0) return kErrDims;
+    TSPLAT_CHECK(ptrs.check(stats, nf24_pack_stats_bytes(out_features, in_features)));
+  }
   const int st = launch_nf24_pack(weight, out_features, in_features, alphabet, alphabet_len,
-                                  base_workspace, code01_t, q2_t, scale,
+                                  base_workspace, code01_t, q2_t, scale, stats,
                                   static_cast<hipStream_t>(stream));
   if (st == kErrLaunch) (void)note(hipErrorLaunchFailure);
   return st;

@@ -201,10 +201,13 @@ int launch_ab2_update(float* sample, const float* prediction, const float* previ
                       hipStream_t stream);
 
 // NF24 packer: w [out_f, in_f] fp32 -> code01_t [in_f, out_f], q2_t, scale
-// [out_f]; base_tmp [out_f] receives max|w_row| / 127.
+// [out_f]; base_tmp [out_f] receives max|w_row| / 127.  stats, or null:
+// nf24_pack_stats_bytes of device memory whose first 9 doubles receive the
+// error report's figures.
+int64_t nf24_pack_stats_bytes(int out_f, int in_f);
 int launch_nf24_pack(const float* w, int out_f, int in_f, const float* alphabet, int alphabet_len,
                      float* base_tmp, int16_t* code01_t, int8_t* q2_t, float* scale,
-                     hipStream_t stream);
+                     double* stats, hipStream_t stream);
 
 // Exact NF24 decode to fp32: [in_f, out_f] like the codes, or [out_f, in_f]
 // (the nn.Linear weight) when transposed.

@@ -54,6 +54,8 @@ SIGNATURES = {
     "tsplat_gemm_nf24_qkv_direct_async": ([_vp] * 11 + [_i] * 8 + [_vp], _i),
     "tsplat_gemm_nf24_qkv_direct_ex_async": ([_vp] * 11 + [_i] * 11 + [_vp], _i),
     "tsplat_nf24_pack_async": ([_vp, _i, _i, _vp, _i, _vp, _vp, _vp, _vp, _vp], _i),
+    "tsplat_nf24_pack_stats_bytes": ([_i, _i], _i64),
+    "tsplat_nf24_pack_stats_async": ([_vp, _i, _i, _vp, _i, _vp, _vp, _vp, _vp, _vp, _vp], _i),
     "tsplat_nf24_decode_async": ([_vp] * 4 + [_i] * 3 + [_vp], _i),
     "tsplat_nf24_gemm_epilogue_async": ([_vp] * 6 + [_i] * 8 + [_vp, _i64, _i, _vp], _i),
     "tsplat_nf24_gemm_precision_async": ([_vp] * 6 + [_i] * 8 + [_vp, _i64, _i, _i, _vp], _i),

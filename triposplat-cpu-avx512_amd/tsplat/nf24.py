@@ -13,6 +13,7 @@ round-half-up residual digits in radix 4 and 256.
 """
 from __future__ import annotations
 
+import functools
 import math
 from statistics import NormalDist
 
@@ -22,16 +23,20 @@ RESIDUAL_MODE_ID = 4
 FORMAT_NAME = "nf24_i16"
 
 
+@functools.lru_cache(maxsize=1)
+def _nf8_level_table():
+    nd = NormalDist()
+    levels = [nd.inv_cdf((i + 0.5) / 255.0) for i in range(255)]
+    peak = max(abs(x) for x in levels)
+    return tuple(sorted([x / peak for x in levels] + [0.0]))
+
+
 def nf8_levels():
     """The 256 normal-float levels as Python floats (float64): the 255
     quantiles sqrt(2)*erfinv(2p-1) at p = (i + 0.5)/255, scaled so that
     max |level| = 1, plus a second zero, sorted
     (scripts/native_linear_nf8_avx512_patch.py:12-20)."""
-    nd = NormalDist()
-    levels = [nd.inv_cdf((i + 0.5) / 255.0) for i in range(255)]
-    peak = max(abs(x) for x in levels)
-    levels = [x / peak for x in levels] + [0.0]
-    return sorted(levels)
+    return list(_nf8_level_table())
 
 
 def make_nf8_codebook(torch_module):
@@ -54,8 +59,9 @@ def quantize_nf24_i16_per_output_channel(weight, codebook=None):
 
     Returns ([code01_t, q2_t, q2_t], [scale, scale, scale], error) with the
     reference's layout (native_linear_rnf8_avx512_patch.py:75-87).  The
-    packing itself runs in the tsplat_nf24_pack_async kernel; ``error``
-    reports the decoded-weight error against the source weight.
+    packing runs in the tsplat_nf24_pack_stats_async kernels; ``error``
+    reports the decoded-weight error against the source weight, from the same
+    pass and read back once.
     """
     import torch
 
@@ -71,53 +77,40 @@ def quantize_nf24_i16_per_output_channel(weight, codebook=None):
     scale = torch.empty(out_f, dtype=torch.float32, device=device)
     lib = load_library()
     with torch.cuda.device(device):
-        status = lib.tsplat_nf24_pack_async(
+        stats = torch.empty(lib.tsplat_nf24_pack_stats_bytes(out_f, in_f) // 8, dtype=torch.float64, device=device)
+        status = lib.tsplat_nf24_pack_stats_async(
             w.data_ptr(), out_f, in_f, alphabet.data_ptr(), int(alphabet.numel()), base.data_ptr(),
-            code01_t.data_ptr(), q2_t.data_ptr(), scale.data_ptr(), current_stream_handle(device),
+            code01_t.data_ptr(), q2_t.data_ptr(), scale.data_ptr(), stats.data_ptr(), current_stream_handle(device),
         )
-    check_status(status, "tsplat_nf24_pack_async")
-    error = _stage_errors(torch, w, base, alphabet)
+        check_status(status, "tsplat_nf24_pack_stats_async")
+        error = _error_report(stats[:9].tolist(), out_f * in_f, int(alphabet.numel()))
     return [code01_t, q2_t, q2_t], [scale, scale, scale], error
 
 
-def _stage_errors(torch, w, base, alphabet):
+def _error_report(stats, count, alphabet_size):
     """The packer's error report, keys and statistics as the reference's
     (native_linear_rnf8_avx512_patch.py:38-87): the residual left after each
     digit -- the NF8-derived level q0 at the base scale, then the radix-4 and
     radix-1024 corrections -- with its RMSE, max-abs and the count of
     corrections clamped to int8; weight_rmse / weight_max_abs are those of the
-    last residual.  The digits are recomputed here with the same fp32
-    elementwise steps as the packing kernel (the int16 code 4 q0 + q1 does not
-    give the digits back); base is the kernel's max|row| / 127."""
-    b = base[:, None]
-    midpoints = ((alphabet[:-1] + alphabet[1:]) * 0.5).contiguous()
-    q0 = alphabet[torch.bucketize(w / b, midpoints)]
-    r1 = w - q0 * b
-    s1 = b / 4.0
-    q1u = torch.floor(r1 / s1 + 0.5)
-    r2 = r1 - q1u.clamp(-128, 127) * s1
-    s2 = b / 1024.0
-    q2u = torch.floor(r2 / s2 + 0.5)
-    r3 = r2 - q2u.clamp(-128, 127) * s2
-    stages = []
-    for stage, (rem, quantizer, unclamped) in enumerate(
-            ((r1, "nf8_derived_int8_alphabet", None), (r2, "shared_scale_int8_radix4", q1u),
-             (r3, "shared_scale_int8_radix256", q2u)), start=1):
-        stages.append({
-            "stage": stage,
-            "quantizer": quantizer,
-            "residual_rmse": float(torch.sqrt(torch.mean(rem * rem)).item()),
-            "residual_max_abs": float(rem.abs().max().item()),
-            "saturated_values": 0 if unclamped is None else int(((unclamped < -128) | (unclamped > 127)).sum().item()),
-        })
-    weight_rms = float(torch.sqrt(torch.mean(w * w)).item())
+    last residual.  stats: the packing kernel's nine figures."""
+    rms = [math.sqrt(s / count) for s in stats[:4]]
+    clamped = (0, int(stats[7]), int(stats[8]))
+    quantizers = ("nf8_derived_int8_alphabet", "shared_scale_int8_radix4", "shared_scale_int8_radix256")
+    stages = [{
+        "stage": i + 1,
+        "quantizer": quantizers[i],
+        "residual_rmse": rms[i],
+        "residual_max_abs": stats[4 + i],
+        "saturated_values": clamped[i],
+    } for i in range(3)]
     return {
-        "weight_rmse": stages[-1]["residual_rmse"],
-        "weight_max_abs": stages[-1]["residual_max_abs"],
-        "weight_rms": weight_rms,
-        "weight_relative_rmse": stages[-1]["residual_rmse"] / max(weight_rms, 1.0e-30),
+        "weight_rmse": rms[2],
+        "weight_max_abs": stats[6],
+        "weight_rms": rms[3],
+        "weight_relative_rmse": rms[2] / max(rms[3], 1.0e-30),
         "residual_mode": FORMAT_NAME,
-        "nf8_derived_alphabet_size": int(alphabet.numel()),
+        "nf8_derived_alphabet_size": alphabet_size,
         "stages": stages,
         "storage_layout": "int16(q0*4+q1) + int8(q2)",
     }
