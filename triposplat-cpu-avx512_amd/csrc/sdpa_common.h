@@ -225,16 +225,10 @@ __global__ __launch_bounds__(kCombineThreads) void sdpa_combine_kernel(SdpaArgs 
   dst[d] = o * (1.0f / l);
 }
 
-// Launches `main(grid, args)` over the query tiles of kBQ queries.  A last
-// round that would leave CUs idle (tiles % CUs workgroups of a
-// one-workgroup-per-CU shape) is split along the keys instead, so that the
-// tail fills every CU; the partial results are merged by a second kernel.
-// cus = 0 disables the split.
+// Launches `main(grid, args)` over the query tiles of a plan; the partial
+// results of its key ranges are merged by a second kernel.
 template <class Main>
-int launch_tiles(SdpaArgs a, const SdpaParams& p, int kBQ, int kBKV, int cus, hipStream_t stream,
-                 Main&& main) {
-  TilePlan pl;
-  if (!plan_tiles(p.B, p.H, p.Lq, p.Lk, kBQ, kBKV, kD, cus, pl)) return kErrDims;
+int launch_plan(SdpaArgs a, const SdpaParams& p, const TilePlan& pl, int kBQ, hipStream_t stream, Main&& main) {
   note_sdpa_query_tile(kBQ);
   a.full_tiles = (int)pl.full_tiles;
   a.splits = pl.splits;
@@ -265,6 +259,19 @@ int launch_tiles(SdpaArgs a, const SdpaParams& p, int kBQ, int kBKV, int cus, hi
     if (hipGetLastError() != hipSuccess) return kErrLaunch;
   }
   return kOk;
+}
+
+// Launches `main(grid, args)` over the query tiles of kBQ queries.  A last
+// round that would leave CUs idle (tiles % CUs workgroups of a
+// one-workgroup-per-CU shape) is split along the keys instead, so that the
+// tail fills every CU; the partial results are merged by a second kernel.
+// cus = 0 disables the split.
+template <class Main>
+int launch_tiles(const SdpaArgs& a, const SdpaParams& p, int kBQ, int kBKV, int cus, hipStream_t stream,
+                 Main&& main) {
+  TilePlan pl;
+  if (!plan_tiles(p.B, p.H, p.Lq, p.Lk, kBQ, kBKV, kD, cus, pl)) return kErrDims;
+  return launch_plan(a, p, pl, kBQ, stream, main);
 }
 
 }  // namespace

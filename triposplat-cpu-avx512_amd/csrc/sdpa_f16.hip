@@ -43,10 +43,12 @@
 //
 // Measured (16 heads) against the fp32 MFMA kernel: L = 16384 7.88 -> 2.75 ms
 // (400 TFLOP/s), 12294 4.57 -> 1.62 ms, 8194 with a key bias 2.14 -> 0.81 ms,
-// 4096 x 2048 280 -> 143 us, 577 52 -> 39 us.  What bounds it: per 32-key
-// block a wave has 24 MFMAs (768 cycles) and about 100 vector instructions,
-// 16 of them exponentials, and the two phases of a SIMD's waves overlap
-// little.
+// 4096 x 2048 280 -> 143 us, 577 52 -> 39 us.  What bounds it: the fp16 matrix
+// cores at the clock they hold, 1.2 PFLOP/s at L = 16384 where a plain 8192^3
+// fp16 library product reaches 1.11 (waves of 64 queries, which read half the
+// LDS fragments per product, 3.05 against 2.97 ms; wave priorities no change).
+// The 128-query tiles are split along the keys where CUs would idle
+// (plan_key_ranges): 300 x 9000 420 -> 102 us.
 
 #include "sdpa_common.h"
 
@@ -572,8 +574,8 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_f16_kernel(SdpaArgs a, const
 }
 
 template <int kLayout, bool kBias, int kWaves, bool kPre>
-int launch_shape(const SdpaParams& p, hipStream_t stream, int cus, const uint2* maxes, const uintx4* pre) {
-  return launch_tiles(make_args(p), p, kWaves * 32, kTileKeys, cus, stream, [&](dim3 grid, const SdpaArgs& a) {
+int launch_shape(const SdpaParams& p, hipStream_t stream, const TilePlan& pl, const uint2* maxes, const uintx4* pre) {
+  return launch_plan(make_args(p), p, pl, kWaves * 32, stream, [&](dim3 grid, const SdpaArgs& a) {
     hipLaunchKernelGGL((sdpa_f16_kernel<kLayout, kBias, kWaves, kPre>), grid, dim3(kWaves * 64), 0, stream, a,
                        maxes, pre);
   });
@@ -600,8 +602,16 @@ int launch_sized(SdpaParams p, hipStream_t stream) {
   const int64_t ntiles = (p.Lk + kTileKeys - 1) / kTileKeys;
   TilePlan pl;
   if (!plan_tiles(p.B, p.H, p.Lq, p.Lk, wide ? 512 : 128, kTileKeys, kD, wide ? cus : 0, pl)) return kErrDims;
-  const size_t part_bytes = (pl.scratch_bytes + 255) / 256 * 256;
   const size_t max_bytes = (size_t)heads * kMaxParts * sizeof(uint2);
+  // Few queries leave CUs of the 128-query tiles idle: those are split along
+  // the keys, where there is room for the ranges' rows.  (Below kMaxLaunchKeys
+  // every workgroup looks through all of k and v first, whatever its range.)
+  const TilePlan whole = pl;
+  if (!wide && p.Lk >= kMaxLaunchKeys) {
+    plan_key_ranges(p.B, p.H, p.Lq, p.Lk, 128, kTileKeys, kD, cus, pl);
+    if (p.scratch != nullptr && pl.scratch_bytes + 256 + max_bytes > p.scratch_bytes) pl = whole;
+  }
+  const size_t part_bytes = (pl.scratch_bytes + 255) / 256 * 256;
   const size_t image_bytes = (size_t)heads * ntiles * kImageTileBytes<kBias>;
   bool image = wide && p.scratch == nullptr && qtiles >= kPreMinQueryTiles<kLayout> &&
                image_bytes <= kPreMaxImageBytes && heads * ntiles <= 0x7fffffff;
@@ -619,6 +629,7 @@ int launch_sized(SdpaParams p, hipStream_t stream) {
       image = false;
       if (p.Lk >= kMaxLaunchKeys) ws = stream_workspace(stream, part_bytes + max_bytes, kSlotSdpaPartial);
     }
+    if (ws == nullptr && !wide) pl = whole;
     if (ws != nullptr) {
       p.scratch = static_cast<float*>(ws);
       p.scratch_bytes = pl.scratch_bytes;
@@ -636,10 +647,10 @@ int launch_sized(SdpaParams p, hipStream_t stream) {
     hipLaunchKernelGGL((sdpa_f16_presplit_kernel<kLayout, kBias>), dim3((unsigned)(heads * ntiles)),
                        dim3(kPreThreads), 0, stream, a, maxes, img, (int)ntiles);
     if (hipGetLastError() != hipSuccess) return kErrLaunch;
-    return launch_shape<0, kBias, 16, true>(p, stream, cus, maxes, img);
+    return launch_shape<0, kBias, 16, true>(p, stream, pl, maxes, img);
   }
-  if (wide) return launch_shape<kLayout, kBias, 16, false>(p, stream, cus, maxes, nullptr);
-  return launch_shape<kLayout, kBias, 4, false>(p, stream, 0, maxes, nullptr);
+  if (wide) return launch_shape<kLayout, kBias, 16, false>(p, stream, pl, maxes, nullptr);
+  return launch_shape<kLayout, kBias, 4, false>(p, stream, pl, maxes, nullptr);
 }
 
 }  // namespace

@@ -10,7 +10,9 @@
 // 2 * CUs - 1, so on a 256-CU MI355X a plan needs at most 511 * 512 * 66 * 4
 // = 69,074,944 bytes.  The array holds 66 MiB (69,206,016 bytes): every plan
 // of a 256-CU device fits; a call whose plan needs more (a device with more
-// CUs) returns -8 before any launch.
+// CUs) returns -8 before any launch.  Strict calls of few queries and at least
+// 1024 keys split every 128-query tile instead, into at most 6 * CUs pieces
+// (51,904,512 bytes), and run whole where that has no room.
 //
 // Sharing.  One array per GPU, shared by every call on that GPU, whatever the
 // stream.  Nothing in it has to start at zero (each partial row is written

@@ -93,6 +93,43 @@ inline bool plan_tiles(int64_t B, int64_t H, int Lq, int Lk, int kBQ, int kBKV, 
   return true;
 }
 
+// Splits every tile of a plan of the four-wave kernel into key ranges where
+// its workgroups leave CUs idle or unevenly loaded.  Time of the fullest CU,
+// in key tiles of one workgroup alone: its ranges, each with kRangeTiles more
+// (prologue, rows written to scratch), over kPairSpeed when several share it,
+// and kMergeTiles for the merge.  Fitted on 16 heads, 48 to 512 tiles of 16 to
+// 193 key tiles (2.95 us each), where it is within a tenth: 300 x 9000 420 ->
+// 102 us, 1024 x 1024 58 -> 47, 2562 x 2562 207 -> 178; 2048 x 1024 stays
+// whole (62 us, 71 in two ranges).  At most 6 pieces per CU.
+constexpr double kRangeTiles = 2.5, kMergeTiles = 2.5, kPairSpeed = 1.2;
+inline void plan_key_ranges(int64_t B, int64_t H, int Lq, int Lk, int kBQ, int kBKV, int kD, int cus,
+                            TilePlan& pl) {
+  const int64_t n = (Lk + kBKV - 1) / kBKV;
+  auto fullest = [&](int s) {
+    const int64_t pieces = (pl.tiles * s + cus - 1) / cus;
+    const double t = (double)pieces * ((double)((n + s - 1) / s) + (s > 1 ? kRangeTiles : 0.0));
+    return t / (pieces > 1 ? kPairSpeed : 1.0) + (s > 1 ? kMergeTiles : 0.0);
+  };
+  double best = 0.94 * fullest(1);  // a gain the model can tell
+  int s0 = 1;
+  for (int s = 2; s <= 32 && s <= n && pl.tiles * s <= 6 * (int64_t)cus; ++s) {
+    const double t = fullest(s);
+    if (t < best) {
+      best = t;
+      s0 = s;
+    }
+  }
+  if (s0 == 1) return;
+  const int64_t partial = (Lq % kBQ != 0) ? B * H : 0;
+  key_ranges(Lk, kBKV, s0, pl.keys_per_split, pl.splits);
+  pl.keys_per_split_p = pl.keys_per_split;
+  pl.splits_p = pl.splits;
+  pl.full_tiles = 0;
+  pl.pieces_full = (pl.tiles - partial) * pl.splits;
+  pl.pieces = pl.tiles * pl.splits;
+  pl.scratch_bytes = (size_t)pl.pieces * kBQ * (kD + 2) * sizeof(float);
+}
+
 // Whether a caller-provided scratch of `have` bytes holds the plan's pieces
 // (the no-allocation entry point's static array; a plan needing more is
 // refused before any launch).
