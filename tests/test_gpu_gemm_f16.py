@@ -125,3 +125,29 @@ def test_whole_code_range(oracle, cuda, hiplib):
     x = r.standard_normal((M, K)).astype(np.float32)
     b = r.standard_normal(N).astype(np.float32)
     _check(oracle, x, c01, q2, s, b, _run(torch, x, c01, q2, s, b))
+
+
+@pytest.mark.parametrize("M,N", [(40, 64), (300, 1024)])
+def test_ends_of_the_range(oracle, cuda, hiplib, M, N):
+    """Finite results of huge and tiny rows (the decoded weights are small) stay finite and exact."""
+    import torch
+
+    K = 96
+    x, w, _ = seeded_linear(M, M, K, N, w_scale=0.02)
+    b = np.zeros(N, np.float32)
+    c01, q2, s = oracle.quantize_nf24_i16(w)
+    w64 = oracle.decode_nf24(c01, q2, s)
+    y = x.copy()
+    scales = {0: 1e36, 3: 3e37, 9: 1e-30, 20: 1e-33, 35: 6e37}
+    for r, f in scales.items():
+        y[r] *= np.float32(f)
+    y[5] = 0.0
+    y[5, 50] = 3.4e38
+    got = _run(torch, y, c01, q2, s, b)
+    assert np.all(np.isfinite(got))
+    for r in [*scales, 5]:
+        assert stats(got[r:r + 1], gemm_f64(y[r:r + 1], w64, b))["rel_rmse"] < 1e-6, r
+    # any scale of the weights: x w stays at 0.02 N(0, 1)
+    for f in (2.0 ** 100, 2.0 ** -100):
+        got = _run(torch, x * np.float32(1.0 / f), c01, q2, s * np.float32(f), b)
+        assert stats(got, gemm_f64(x, w64, b))["rel_rmse"] < 1e-6, f

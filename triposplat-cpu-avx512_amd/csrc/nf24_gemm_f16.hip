@@ -132,9 +132,6 @@ __device__ __forceinline__ float row_scale(uint32_t mx_bits) {
   const int field = 260 - (int)(mx_bits >> 23);  // exponent field of 2^(6 - e)
   return mx_bits == 0 ? 1.0f : __uint_as_float((uint32_t)min(max(field, 1), 253) << 23);
 }
-__device__ __forceinline__ float inverse_pow2(float s) {
-  return __uint_as_float((254u << 23) - __float_as_uint(s));
-}
 
 // Largest of x over eight lanes (a swizzle has no lane addresses to hold, and
 // so none that the QKV epilogue would share and keep over the K loop).
@@ -482,14 +479,19 @@ void nf24_gemm_f16_kernel(GemmArgs a) {
   const int row_e = (wave_e / C::WN) * C::kTM, col_e = (wave_e % C::WN) * C::kTN;
   const int g_e = (tid_e >> 5) & 1, l_e = tid_e & 31;
 
-  // out before the epilogue: bias + acc * (256 / s) * scale, a row block at a
-  // time (all the row scales at once would spill)
-  float bv[C::kNB], sc[C::kNB];
+  // out before the epilogue, a row block at a time (all the row scales at once
+  // would spill): bias + acc * (256 / s) * scale, the powers of two applied to
+  // acc together, before scale's fraction in [1, 2): nothing on the way to the
+  // result is larger than it, or rounded before it.
+  float bv[C::kNB], frac[C::kNB];
+  int expo[C::kNB];
 #pragma unroll
   for (int nb = 0; nb < C::kNB; ++nb) {
     const int col = c0 + col_e + nb * 32 + l_e;
+    const float sc = col < a.n_count ? a.scale[a.n_start + col] : 0.0f;
     bv[nb] = col < a.n_count ? a.bias[a.n_start + col] : 0.0f;
-    sc[nb] = col < a.n_count ? 256.0f * a.scale[a.n_start + col] : 0.0f;
+    frac[nb] = 2.0f * __builtin_amdgcn_frexp_mantf(sc);
+    expo[nb] = __builtin_amdgcn_frexp_expf(sc) + (8 - 1 + 127);
   }
 #pragma unroll
   for (int mb = 0; mb < C::kMB; ++mb) {
@@ -499,8 +501,10 @@ void nf24_gemm_f16_kernel(GemmArgs a) {
 #pragma unroll
       for (int e = 0; e < 4; ++e)
 #pragma unroll
-        for (int nb = 0; nb < C::kNB; ++nb)
-          acc[mb][nb][4 * r4 + e] = fmaf(acc[mb][nb][4 * r4 + e] * inverse_pow2(rs[e]), sc[nb], bv[nb]);
+        for (int nb = 0; nb < C::kNB; ++nb) {
+          const float t = __builtin_amdgcn_ldexpf(acc[mb][nb][4 * r4 + e], expo[nb] - (int)(__float_as_uint(rs[e]) >> 23));
+          acc[mb][nb][4 * r4 + e] = fmaf(t, frac[nb], bv[nb]);
+        }
     }
     __builtin_amdgcn_sched_barrier(0);
   }
