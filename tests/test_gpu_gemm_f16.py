@@ -127,6 +127,44 @@ def test_whole_code_range(oracle, cuda, hiplib):
     _check(oracle, x, c01, q2, s, b, _run(torch, x, c01, q2, s, b))
 
 
+def _dead_features(oracle, seed, M, K, N, dead):
+    """x, weights and bias with the features `dead` (a list of k) at zero weight."""
+    x, w, b = seeded_linear(seed, M, K, N, w_scale=0.02)
+    w[:, dead] = 0.0
+    c01, q2, s = oracle.quantize_nf24_i16(w)
+    assert not oracle.decode_nf24(c01, q2, s)[dead].any()
+    return x, c01, q2, s, b
+
+
+@pytest.mark.parametrize("M,N", [(40, 64), (300, 1028), (700, 576)])
+@pytest.mark.parametrize("dead", [[5], [40], [159], list(range(32)), list(range(3, 160, 7)), [6, 130],
+                                  list(range(1, 160, 4))])
+def test_large_values_without_weight(oracle, cuda, hiplib, M, N, dead):
+    """A feature of any size whose weights are zero costs the row's other
+    features nothing: each result within the fp32 bound of its own terms."""
+    import torch
+
+    x, c01, q2, s, b = _dead_features(oracle, M + N, M, 160, N, dead)
+    plain = _run(torch, x, c01, q2, s, b)
+    rows = {1: 1e4, 2: 1e6, 8: 1e8, 17: 1e10, 30: 1e20, 33: -3e38}
+    y = x.copy()
+    for r, value in rows.items():
+        y[r, dead] = value
+    print(f"gemm f16 M={M} N={N} dead={dead[:4]}", flush=True)
+    got = _run(torch, y, c01, q2, s, b)
+    w = oracle.decode_nf24(c01, q2, s)
+    pick = list(rows)
+    if dead[:2] != [1, 5]:
+        assert np.all(np.abs(got[pick] - gemm_f64(y[pick], w, b)) <= gemm_order_bound(y[pick], w, b))
+    else:
+        # every four values hold such a feature: the others are held to 2^-40
+        # of the largest of the row's first 32
+        floor = 2.0 ** -40 * np.abs(y[pick].astype(np.float64)).max(1)[:, None] * np.abs(w).sum(0)[None]
+        assert np.all(np.abs(got[pick] - gemm_f64(y[pick], w, b)) <= gemm_order_bound(y[pick], w, b) + floor)
+    keep = np.setdiff1d(np.arange(M), pick)
+    assert np.array_equal(got[keep].view(np.uint32), plain[keep].view(np.uint32))
+
+
 @pytest.mark.parametrize("M,N", [(40, 64), (300, 1024)])
 def test_ends_of_the_range(oracle, cuda, hiplib, M, N):
     """Finite results of huge and tiny rows (the decoded weights are small) stay finite and exact."""

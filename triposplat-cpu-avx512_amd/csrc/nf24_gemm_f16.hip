@@ -4,7 +4,8 @@
 // fp32 MFMA peaks at 157 TFLOP/s on this part, fp16 MFMA at sixteen times
 // that, so each fp32 operand is carried as two fp16 values and each product
 // as three fp16 products with fp32 accumulation:
-//   x * s = xh + xl,  p / 256 = wh + wl,  acc = sum xh*wh + xh*wl + xl*wh,
+//   x * s = xh + 2^-11 xl,  p / 256 = wh + wl,
+//   acc = sum xh*wh + xh*wl + xl*(2^-11 wh),
 //   out = bias + acc * (256 / s) * scale[n]
 // with p = (int32)code01 * 256 + q2 the integer payload (the reference's
 // decode, scripts/gemm_nf24_i16_avx512.c:26-33, is fp32(p) * scale[n]) and s
@@ -14,25 +15,35 @@
 //     for every code the format can hold, and exactly for |p| < 2^22 (the
 //     packer's payloads stay below 2^17).  scale[n] is applied once, to the
 //     sum.
-//   * x: xh + xl holds x * s to within one unit of fp32's last place as long
-//     as |x| is above 2^-24 of the row's scale; below that the error is at
-//     most 2^-25 / s, i.e. 2^-31 of the largest value the scale was set from.
+//   * x: the pair holds x * s to within one unit of fp32's last place from
+//     2^-13 on, and to 2^-36 below: xl is kept 2^11 times larger, so that it
+//     does not run out of fp16's range with xh, and meets a copy of wh taken
+//     down by as much (exact: wh is a multiple of 2^-8).
 //   * the dropped xl*wl is below 2^-22 of the product (2^-24 rms).
 // Products of fp16 values are exact in fp32, and the matrix core rounds its
 // accumulator twice per 16 k and term instead of once per k, so the error
 // against 64 bits is below the fp32 MFMA kernel's (N(0, 1) x, K = 1024:
 // 3.6e-7 against 5.7e-7 relative).
 //
-// Row scale.  s brings the largest of the row's first 32 values (all of
-// them, when those are zero) to [2^6, 2^7): 2^9 of headroom below fp16's
-// largest value.  It depends on that row alone, so a row's result does not
-// depend on the rows it shares a tile with.  A larger value further along the
-// row makes xh infinite and with it the row's sums; the workgroup sees that
-// in its accumulators, sets the scale of those rows from a scan of the whole
-// row and runs the K loop once more, with xh held to +-65504: an infinity or
-// NaN of x itself is then one in xl, which meets wh alone, and the sums are
-// what fp32 products would give, an infinity of the products' sign, or NaN
-// where wh is zero or the signs disagree.
+// Row scale.  s brings the largest of the row's first 32 values (of all of
+// them, when those are zero) to [2^3, 2^4): 2^12 of headroom, and as much
+// below for values that matter beside weights which are zero for the large
+// ones.  The pairs of a row do not serve where |x * s| reaches fp16's infinity
+// (the workgroup sees that in its accumulators), or where the largest of four
+// neighbouring values is less than 2^-17 and not zero (seen while staging):
+// their pairs would hold less than 2^-19 of it.  Such rows are found by a scan,
+// get a scale from the whole row (largest value to [2^14, 2^15)) and the
+// workgroup runs its K loop once more; rows whose values spread too far for
+// that as well, or are not all finite, are then summed as fp32 products.  All
+// of this depends on the row alone, so a row's result does not depend on the
+// rows it shares a tile with.  What the pairs lose is at most 2^-36 / s of a
+// value, 2^-39 of the row's largest, beside values that large in its group of
+// four.
+//
+// A call pays for such rows with the second pass: 4096 x 1024 x 3072 with one
+// value of 1e6 80 -> 180 us (fp32 tiles: 196), a feature 3000 times the others
+// 213, 1e5 times 262; 600 times, in the first pass, 90 (with a headroom of 2^9
+// and without the shift of xl: 197).
 //
 // Tiling: BM x BN workgroup tile, WM x WN waves, a wave owns MB x NB blocks
 // of 32 x 32 (the accumulator layout the epilogues of nf24_gemm_common.h
@@ -47,15 +58,16 @@
 // loaded a step earlier, and the step after that is loaded into them, so no
 // wave waits for memory inside a step.  (Staged after the MFMAs instead, from
 // loads of the same step: 4096 x 1024 x 3072 84 us, 12294 x 4096 x 1024 350,
-// fused QKV over 8194 rows 261, 600 x 1024 x 1024 34.)
+// fused QKV over 8194 rows 261, 600 x 1024 x 1024 34.)  The check of each four
+// values and the shifted copy of wh cost 2 to 3 % of the larger calls.
 //
-// Measured against the fp32 MFMA tiles: 4096 x 1024 x 3072 197 -> 78 us (330
-// TFLOP/s), 12294 x 4096 x 1024 788 -> 284 us (363), 12294 x 1024 x 4096 765 ->
-// 299 us, fused QKV over 8194 rows 496 -> 233 us, 600 x 1024 x 1024 47 -> 32
-// us.  What bounds it: the fp16 matrix cores at the clock they hold; three
-// products at 363 TFLOP/s are 1.09 PFLOP/s, a plain 8192^3 fp16 library product
-// on the same card 1.11.  Grids of one round or less are bound by a tile's
-// chain of K steps instead (31 us at K = 1024 for the smallest).
+// Measured against the fp32 MFMA tiles: 4096 x 1024 x 3072 197 -> 79 us (326
+// TFLOP/s), 12294 x 4096 x 1024 gated 817 -> 319 us (323), fused QKV over 8194
+// rows 496 -> 243 us, 600 x 1024 x 1024 47 -> 27 us.  What bounds it: the fp16
+// matrix cores at the clock they hold; three products at 326 TFLOP/s are 0.98
+// PFLOP/s, a plain 8192^3 fp16 library product on the same card 1.11.  Grids of
+// one round or less are bound by a tile's chain of K steps instead (27 us at
+// K = 1024 for the smallest).
 
 #include "nf24_gemm_common.h"
 
@@ -104,10 +116,22 @@ __device__ __forceinline__ floatx16 mfma_f16(const half8& a, const half8& b, flo
 
 // (hi, lo) fp16 pairs of a and b: hi = fp16(v), lo = fp16(v - hi), the
 // difference exact in fp32.
-__device__ __forceinline__ void split2(float a, float b, float hi_a, float hi_b, unsigned& hi, unsigned& lo) {
-  const half2v h = __builtin_convertvector(floatx2{hi_a, hi_b}, half2v);
+__device__ __forceinline__ void split2(float a, float b, unsigned& hi, unsigned& lo) {
+  const half2v h = __builtin_convertvector(floatx2{a, b}, half2v);
   hi = __builtin_bit_cast(unsigned, h);
   lo = __builtin_bit_cast(unsigned, __builtin_convertvector(floatx2{a - (float)h[0], b - (float)h[1]}, half2v));
+}
+// The same of x[i] * s for a power of two s, given v = x * s, with lo kLoShift
+// times larger.  (Each step an instruction: x * s - hi and its shift are mixed
+// fp32 / fp16 FMAs.)
+constexpr int kLoShift = 2048;
+__device__ __forceinline__ void split2_shifted(const floatx4& x, const floatx4& v, float s, int i, unsigned& hi,
+                                               unsigned& lo) {
+  const half2v h = __builtin_convertvector(floatx2{v[i], v[i + 1]}, half2v);
+  hi = __builtin_bit_cast(unsigned, h);
+  const half2v l = {(_Float16)fmaf(fmaf(x[i], s, -(float)h[0]), (float)kLoShift, 0.0f),
+                    (_Float16)fmaf(fmaf(x[i + 1], s, -(float)h[1]), (float)kLoShift, 0.0f)};
+  lo = __builtin_bit_cast(unsigned, l);
 }
 
 // p / 256 of column e of a staged unit row (two int16 codes per word, four
@@ -126,19 +150,78 @@ __device__ __forceinline__ void store_pairs(_Float16* dst, const unsigned (&w)[N
   else *reinterpret_cast<unsigned*>(dst) = w[0];
 }
 
-// Row scale from the bits of the row's largest magnitude: the power of two
-// that brings it to [2^6, 2^7), with a normal reciprocal.
+// A row's pairs serve where |x * s| stays below kRowTop (fp16's infinity) and
+// the largest of each four values (a staging unit) that are not all zero
+// reaches kUnitMin.
+constexpr float kRowTop = 65520.0f;
+constexpr uint32_t kUnitMin = (127u - 17u) << 23;  // bits of 2^-17
+
+// The power of two that brings a magnitude (as bits) to [2^kTop, 2^(kTop + 1)),
+// with a normal reciprocal.
+constexpr int kFirstTop = 3;   // the largest of the row's first 32 values
+constexpr int kWholeTop = 14;  // the largest of the row
+template <int kTop>
 __device__ __forceinline__ float row_scale(uint32_t mx_bits) {
-  const int field = 260 - (int)(mx_bits >> 23);  // exponent field of 2^(6 - e)
+  const int field = 254 + kTop - (int)(mx_bits >> 23);  // exponent field of 2^(kTop - e)
   return mx_bits == 0 ? 1.0f : __uint_as_float((uint32_t)min(max(field, 1), 253) << 23);
 }
 
-// Largest of x over eight lanes (a swizzle has no lane addresses to hold, and
-// so none that the QKV epilogue would share and keep over the K loop).
+// Largest of x over eight lanes (lane ^ 1, ^ 2, then the row's halves
+// mirrored).
 __device__ __forceinline__ uint32_t max8(uint32_t x) {
-  x = max(x, (uint32_t)__builtin_amdgcn_ds_swizzle((int)x, (1 << 10) | 0x1f));  // lane ^ 1
-  x = max(x, (uint32_t)__builtin_amdgcn_ds_swizzle((int)x, (2 << 10) | 0x1f));
-  return max(x, (uint32_t)__builtin_amdgcn_ds_swizzle((int)x, (4 << 10) | 0x1f));
+  x = max(x, (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0xb1, 0xf, 0xf, true));
+  x = max(x, (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x4e, 0xf, 0xf, true));
+  return max(x, (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x141, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float max_abs(const floatx4& v) {
+  return fmaxf(fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fabsf(v[2])), fabsf(v[3]));
+}
+
+// bias + x * decode(W) in fp32 products for a block of 32 rows, the lane's row
+// `row` (in range), and the wave's columns from col0: sums in the accumulator
+// layout, straight from memory (rare: no tile is shared).
+template <class C>
+__device__ __forceinline__ void fp32_rows(const GemmArgs& a, int row, int col0, int g, int l32,
+                                          floatx16 (&sum)[C::kNB]) {
+  // kTurn k a turn for each half (half g on k0 + kTurn * g ..): a turn's loads
+  // are in flight together, and no more of them than the registers beside the
+  // tile's accumulators hold
+  constexpr int kTurn = C::kMinWaves <= 2 ? 8 : 4;
+  float sc[C::kNB];
+#pragma unroll
+  for (int nb = 0; nb < C::kNB; ++nb) {
+    const int col = min(col0 + nb * 32 + l32, a.n_count - 1);
+    sc[nb] = a.scale[a.n_start + col];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) sum[nb][r] = a.bias[a.n_start + col];
+  }
+#pragma unroll 1
+  for (int k0 = kTurn * g; k0 - kTurn * g < a.K; k0 += 2 * kTurn) {
+    const float* x = a.x + (int64_t)row * a.stride_x;
+    float xv[kTurn];
+    int c[kTurn][C::kNB], q[kTurn][C::kNB];
+#pragma unroll
+    for (int i = 0; i < kTurn; ++i) {
+      const int k = min(k0 + i, a.K - 1);
+      xv[i] = x[k];
+      const int64_t w = (int64_t)k * a.N + a.n_start;
+#pragma unroll
+      for (int nb = 0; nb < C::kNB; ++nb) {
+        const int64_t o = w + min(col0 + nb * 32 + l32, a.n_count - 1);
+        c[i][nb] = a.code01[o];
+        q[i][nb] = a.q2[o];
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < kTurn; ++i) {
+      const bool in = k0 + i < a.K;
+#pragma unroll
+      for (int nb = 0; nb < C::kNB; ++nb)
+        sum[nb] = __builtin_amdgcn_mfma_f32_32x32x2f32(
+            in ? xv[i] : 0.0f, in ? (float)(c[i][nb] * 256 + q[i][nb]) * sc[nb] : 0.0f, sum[nb], 0, 0, 0);
+    }
+  }
 }
 
 // kVec: x rows 16-byte aligned with K % 4 == 0; N, n_start, n_count
@@ -151,8 +234,8 @@ void nf24_gemm_f16_kernel(GemmArgs a) {
   __shared__ __attribute__((aligned(16))) _Float16 xs[2][2][C::BM * C::BK];  // [buffer][hi, lo]
   __shared__ __attribute__((aligned(16))) _Float16 ws[2][2][C::BN * C::BK];
   __shared__ __attribute__((aligned(16))) float row_sc[C::BM];  // s of each row
-  __shared__ uint8_t row_flag[C::BM];  // the first pass left the row without finite sums
-  __shared__ int second;
+  __shared__ uint8_t row_flag[C::BM];  // the row's pairs do not serve
+  __shared__ int second;               // the scales are those of the second pass
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -264,8 +347,7 @@ void nf24_gemm_f16_kernel(GemmArgs a) {
 
   // A step's staging in kStages parts: x unit j, then column e of W unit j.
   // A part places its values in LDS buffer buf and, its registers free, loads
-  // the step at k_next into them.  limit: bound of xh, infinite in the first
-  // pass.
+  // the step at k_next into them.
   // LDS positions: x units of a thread are a multiple of 16 rows apart, and
   // the four columns of a W unit (w_col a multiple of 4) are rows whose two
   // low bits alone differ.
@@ -277,17 +359,18 @@ void nf24_gemm_f16_kernel(GemmArgs a) {
   for (int j = 0; j < C::kWIter; ++j) w_dst[j] = chunk_offset(w_row(w_col[j]), w_k[j] >> 3) + (w_k[j] & 7);
   constexpr int kStages = C::kXIter + 4 * C::kWIter;
   float rsc[C::kXIter];  // scale of x unit j's row
-  auto stage = [&](int part, int buf, float limit, int k_next) {
+  // bits of the smallest of its units' maxima so far, less one (so that a
+  // maximum of zero is the largest of all)
+  uint32_t low = 0xffffffffu;
+  auto stage = [&](int part, int buf, int k_next) {
     if (part < C::kXIter) {
       const int j = part;
       if (!x_unit(j)) return;
       const floatx4 v = xr[j] * rsc[j];
-      float m[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) m[e] = __builtin_amdgcn_fmed3f(v[e], -limit, limit);
+      low = min(low, __float_as_uint(max_abs(v)) - 1u);
       unsigned hi[2], lo[2];
-      split2(v[0], v[1], m[0], m[1], hi[0], lo[0]);
-      split2(v[2], v[3], m[2], m[3], hi[1], lo[1]);
+      split2_shifted(xr[j], v, rsc[j], 0, hi[0], lo[0]);
+      split2_shifted(xr[j], v, rsc[j], 2, hi[1], lo[1]);
       const int off = x_dst + j * (C::kThreads / (C::BK / 4)) * 32;
       store_pairs(&xs[buf][0][off], hi);
       store_pairs(&xs[buf][1][off], lo);
@@ -300,7 +383,7 @@ void nf24_gemm_f16_kernel(GemmArgs a) {
       for (int i = 0; i < C::WK / 2; ++i) {
         const float p0 = w_payload(cr[j][2 * i], qr[j][2 * i] ^ kFlipQ2, e);
         const float p1 = w_payload(cr[j][2 * i + 1], qr[j][2 * i + 1] ^ kFlipQ2, e);
-        split2(p0, p1, p0, p1, hi[i], lo[i]);
+        split2(p0, p1, hi[i], lo[i]);
       }
       const int off = w_dst[j] ^ (e * 32);
       store_pairs(&ws[buf][0][off], hi);
@@ -309,22 +392,52 @@ void nf24_gemm_f16_kernel(GemmArgs a) {
     }
   };
 
-  // Largest magnitude (as bits) among the values from k0 on of the row of x
-  // unit idx, over the row's eight lanes (plain loads: this is rare).
-  auto row_max = [&](int idx, int k0) {
+  // Largest magnitude (as bits) of the row of x unit idx, over the row's eight
+  // lanes (plain loads: this is rare).
+  auto row_max = [&](int idx) {
     const int row = min(idx / (C::BK / 4), rows - 1);
-    const float* src = a.x + (int64_t)(m0 + row) * a.stride_x + 4 * (idx % (C::BK / 4));
+    const float* src = a.x + (int64_t)(m0 + row) * a.stride_x;
     uint32_t mx = 0;
 #pragma unroll 1
-    for (int k = k0; k < a.K; k += C::BK)
+    for (int k = 4 * (idx % (C::BK / 4)); k < a.K; k += 4 * C::BK)
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (k + 4 * (idx % (C::BK / 4)) + e < a.K) mx = max(mx, __float_as_uint(src[k + e]) & 0x7fffffffu);
-    mx = max8(mx);
-    return mx;
+      for (int i = 0; i < 16; ++i)
+        mx = max(mx, __float_as_uint(src[min(k + i / 4 * C::BK + i % 4, a.K - 1)]) & 0x7fffffffu);
+    return max8(mx);
   };
-  auto set_scale = [&](int idx, uint32_t mx) {
-    if (idx < C::kXUnits && idx % (C::BK / 4) == 0) row_sc[idx / (C::BK / 4)] = row_scale(mx);
+  auto set_scale = [&](int idx, float scale) {
+    if (idx < C::kXUnits && idx % (C::BK / 4) == 0) row_sc[idx / (C::BK / 4)] = scale;
+  };
+  // row_flag: the rows whose pairs under the present scales do not serve.
+  auto find_rows = [&](int first) {
+#pragma unroll 1
+    for (int idx = first; idx < C::kXUnits; idx += C::kThreads) {
+      const int row = idx / (C::BK / 4), kc = idx % (C::BK / 4);
+      const float* src = a.x + (int64_t)(m0 + min(row, rows - 1)) * a.stride_x;
+      const float s = row_sc[row];
+      bool bad = false;
+#pragma unroll 1
+      for (int k = 4 * kc; k < a.K; k += 4 * C::BK) {
+        float v[4][4];  // four units' loads in flight
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[u][e] = src[min(k + u * C::BK + e, a.K - 1)];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          uint32_t mx = 0;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float w = k + u * C::BK + e < a.K ? fabsf(v[u][e] * s) : 0.0f;
+            bad |= !(w < kRowTop);
+            mx = max(mx, __float_as_uint(w));
+          }
+          bad |= mx - 1u < kUnitMin - 1u;
+        }
+      }
+      const uint32_t any = max8(bad ? 1u : 0u);
+      if (kc == 0) row_flag[row] = row < rows && any != 0;
+    }
   };
 
   // vector ALU instructions between two MFMAs of a step: the staging's share
@@ -351,10 +464,10 @@ void nf24_gemm_f16_kernel(GemmArgs a) {
     const int idx = tid + j * C::kThreads;
     const bool zero = mx == 0 && x_unit(j) && idx / (C::BK / 4) < rows;
     if (__builtin_amdgcn_ballot_w64(zero) != 0) {
-      const uint32_t rest = row_max(idx, C::BK);
+      const uint32_t rest = row_max(idx);
       if (mx == 0) mx = rest;
     }
-    set_scale(idx, mx);
+    set_scale(idx, row_scale<kFirstTop>(mx));
   }
   // `second` lives in LDS, where the compiler does not know it: one K loop in
   // the code for both passes, the second being the exception.
@@ -363,9 +476,9 @@ void nf24_gemm_f16_kernel(GemmArgs a) {
   // One K step on LDS buffer P: 2 * kMB groups of MFMAs (16 k, one row block),
   // each with the fragment reads of the next group and, in all but the last
   // step, a share of the next step's staging between its MFMAs.
-  auto step = [&](auto staged, int P, float limit, int k_next) {
+  auto step = [&](auto staged, int P, int k_next) {
     constexpr int kGroups = 2 * C::kMB;
-    half8 ah[2], al[2], bh[2][C::kNB], bl[2][C::kNB];
+    half8 ah[2], al[2], bh[2][C::kNB], bl[2][C::kNB], bs[C::kNB];
     auto read_a = [&](int grp) {
       const int off = (a_src ^ (grp / C::kMB * 16)) + grp % C::kMB * 32 * 32;
       ah[grp & 1] = lds_frag(&xs[P][0][off]);
@@ -400,28 +513,42 @@ void nf24_gemm_f16_kernel(GemmArgs a) {
       for (int nb = 0; nb < C::kNB; ++nb) acc[mb][nb] = mfma_f16(ah[grp & 1], bh[s][nb], acc[mb][nb]);
 #pragma unroll
       for (int nb = 0; nb < C::kNB; ++nb) acc[mb][nb] = mfma_f16(ah[grp & 1], bl[s][nb], acc[mb][nb]);
+      if (mb == 0) {
 #pragma unroll
-      for (int nb = 0; nb < C::kNB; ++nb) acc[mb][nb] = mfma_f16(al[grp & 1], bh[s][nb], acc[mb][nb]);
-      if constexpr (decltype(staged)::value) {
-#pragma unroll
-        for (int u = grp * kStages / kGroups; u < (grp + 1) * kStages / kGroups; ++u)
-          stage(u, P ^ 1, limit, k_next);
-        // an MFMA, then what fits beside it (mask 8: MFMA, 2: vector ALU)
-#pragma unroll
-        for (int i = 0; i < 3 * C::kNB; ++i) {
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x002, kStageAlu, 0);
-        }
+        for (int nb = 0; nb < C::kNB; ++nb) bs[nb] = bh[s][nb] * (_Float16)(1.0f / kLoShift);
       }
+      auto share = [&](int first, int end, int mfmas) {
+        if constexpr (decltype(staged)::value) {
+#pragma unroll
+          for (int u = first; u < end; ++u) stage(u, P ^ 1, k_next);
+          // an MFMA, then what fits beside it (mask 8: MFMA, 2: vector ALU)
+#pragma unroll
+          for (int i = 0; i < mfmas; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, kStageAlu, 0);
+          }
+        }
+      };
+      const int first = grp * kStages / kGroups, end = (grp + 1) * kStages / kGroups;
+      if (mb == 0) {
+        // (apart, or the products that wait for bs are chained behind it)
+        share(first, end, 2 * C::kNB);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int nb = 0; nb < C::kNB; ++nb) acc[mb][nb] = mfma_f16(al[grp & 1], bs[nb], acc[mb][nb]);
+      if (mb != 0) share(first, end, 3 * C::kNB);
       __builtin_amdgcn_sched_barrier(0);
     }
   };
+  bool rest = false;  // some rows' pairs serve under neither scale
   for (;;) {
-    const float limit = __builtin_amdgcn_readfirstlane(second) != 0 ? 65504.0f : INFINITY;
+    int tid_x = tid;  // (addresses that are not kept over the K loop)
+    asm volatile("" : "+v"(tid_x));
 #pragma unroll
-    for (int j = 0; j < C::kXIter; ++j) rsc[j] = row_sc[x_unit(j) ? (tid + j * C::kThreads) / (C::BK / 4) : 0];
+    for (int j = 0; j < C::kXIter; ++j) rsc[j] = row_sc[x_unit(j) ? (tid_x + j * C::kThreads) / (C::BK / 4) : 0];
 #pragma unroll
-    for (int u = 0; u < kStages; ++u) stage(u, 0, limit, min(1, nk - 1) * C::BK);
+    for (int u = 0; u < kStages; ++u) stage(u, 0, min(1, nk - 1) * C::BK);
     __syncthreads();
 #pragma unroll
     for (int mb = 0; mb < C::kMB; ++mb)
@@ -431,11 +558,10 @@ void nf24_gemm_f16_kernel(GemmArgs a) {
         for (int r = 0; r < 16; ++r) acc[mb][nb][r] = 0.0f;
     for (int kt = 0; kt + 1 < nk; ++kt) {
       // (the last staged step loads its own tile again, unused)
-      step(std::true_type{}, kt & 1, limit, min(kt + 2, nk - 1) * C::BK);
+      step(std::true_type{}, kt & 1, min(kt + 2, nk - 1) * C::BK);
       __syncthreads();
     }
-    step(std::false_type{}, (nk - 1) & 1, limit, 0);
-    __syncthreads();
+    step(std::false_type{}, (nk - 1) & 1, 0);
     // 0 * acc is NaN for an accumulator that is not finite
     float chk = 0.0f;
 #pragma unroll
@@ -444,30 +570,26 @@ void nf24_gemm_f16_kernel(GemmArgs a) {
       for (int nb = 0; nb < C::kNB; ++nb)
 #pragma unroll
         for (int r = 0; r < 16; ++r) chk = fmaf(acc[mb][nb][r], 0.0f, chk);
-    if (!__builtin_amdgcn_readfirstlane(__syncthreads_or(chk != 0.0f))) break;
-    if (__builtin_amdgcn_readfirstlane(second) != 0) break;
-    // Scales of the rows with such sums from the whole row, and once more.
-    for (int i = tid; i < C::BM; i += C::kThreads) row_flag[i] = 0;
+    if (!__builtin_amdgcn_readfirstlane(__syncthreads_or(chk != 0.0f || low < kUnitMin - 1u))) break;
+    rest = __builtin_amdgcn_readfirstlane(second) != 0;
+    asm volatile("" : "+v"(tid_x));
+    find_rows(tid_x);
     __syncthreads();
+    if (rest) break;
+    // Those rows' scales from the whole row, and once more (the other rows' sums
+    // come out as they were).
     if (tid == 0) second = 1;
-#pragma unroll
-    for (int mb = 0; mb < C::kMB; ++mb)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        bool bad = false;
-#pragma unroll
-        for (int nb = 0; nb < C::kNB; ++nb) bad |= !(fabsf(acc[mb][nb][r]) < INFINITY);
-        if (bad) row_flag[wm * C::kTM + mb * 32 + 8 * (r / 4) + 4 * g + r % 4] = 1;
-      }
-    __syncthreads();
 #pragma unroll 1
-    for (int idx = tid; idx < C::kXUnits; idx += C::kThreads) {
+    for (int idx = tid_x; idx < C::kXUnits; idx += C::kThreads) {
       const bool flagged = row_flag[idx / (C::BK / 4)] != 0;
       if (__builtin_amdgcn_ballot_w64(flagged) == 0) continue;
-      const uint32_t mx = row_max(idx, 0);
-      if (flagged) set_scale(idx, mx);
+      const uint32_t mx = row_max(idx);
+      if (flagged) set_scale(idx, row_scale<kWholeTop>(mx));
     }
-    load_tile(0);
+    low = 0xffffffffu;
+    int k_first = 0;  // (a step of its own, for the addresses)
+    asm volatile("" : "+s"(k_first));
+    load_tile(k_first);
   }
 
   // The wave's coordinates again, from a copy of the thread index that the
@@ -509,10 +631,33 @@ void nf24_gemm_f16_kernel(GemmArgs a) {
     __builtin_amdgcn_sched_barrier(0);
   }
 
+  if (rest) {
+    // The sums of the rows left over, as fp32 products.
+#pragma unroll 1
+    for (int mb = 0; mb < C::kMB; ++mb) {
+      const int row_b = row_e + mb * 32;
+      if (__builtin_amdgcn_ballot_w64(row_flag[row_b + l_e] != 0) == 0) continue;
+      floatx16 sum[C::kNB];
+      fp32_rows<C>(a, m0 + min(row_b + l_e, rows - 1), c0 + col_e, g_e, l_e, sum);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const bool take = row_flag[row_b + 8 * (r / 4) + 4 * g_e + r % 4] != 0;
+#pragma unroll
+        for (int m = 0; m < C::kMB; ++m)
+#pragma unroll
+          for (int nb = 0; nb < C::kNB; ++nb)
+            acc[m][nb][r] = take && m == mb ? sum[nb][r] : acc[m][nb][r];
+      }
+    }
+  }
+
+  asm volatile("" : "+v"(tid_e));
+  const int wave_s = __builtin_amdgcn_readfirstlane(tid_e >> 6);
+  const int row_s = m0 + (wave_s / C::WN) * C::kTM, col_s = c0 + (wave_s % C::WN) * C::kTN;
   if constexpr (kEpi == kEpiQkv) {
-    qkv_epilogue<C>(a, acc, m0 + row_e, c0 + col_e, g_e, l_e);
+    qkv_epilogue<C>(a, acc, row_s, col_s, (tid_e >> 5) & 1, tid_e & 31);
   } else {
-    store_result<C::kMB, C::kNB, kEpi>(a, acc, m0 + row_e, c0 + col_e, g_e, l_e);
+    store_result<C::kMB, C::kNB, kEpi>(a, acc, row_s, col_s, (tid_e >> 5) & 1, tid_e & 31);
   }
 }
 
