@@ -189,3 +189,21 @@ def test_ends_of_the_range(oracle, cuda, hiplib, M, N):
     for f in (2.0 ** 100, 2.0 ** -100):
         got = _run(torch, x * np.float32(1.0 / f), c01, q2, s * np.float32(f), b)
         assert stats(got, gemm_f64(x, w64, b))["rel_rmse"] < 1e-6, f
+
+
+@pytest.mark.parametrize("M", [37, 300])
+@pytest.mark.parametrize("K,N", [(96, 130), (100, 131), (98, 132), (96, 252)])
+def test_ranges_of_any_alignment(oracle, cuda, hiplib, M, K, N):
+    """A column range of a small call holds the bits of the whole call, whichever
+    kernel the weight's sizes send it to."""
+    import torch
+    from tsplat.nf24 import nf24_linear
+
+    x, w, b = seeded_linear(M + K + N, M, K, N, w_scale=0.02)
+    c01, q2, s = oracle.quantize_nf24_i16(w)
+    _check(oracle, x, c01, q2, s, b, _run(torch, x, c01, q2, s, b))
+    t = [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (x, c01, q2, s, b)]
+    full = nf24_linear(*t)
+    for start, count in ((0, 2), (2, 6), (5, 7), (4, 100), (N - 1, 1), (1, N - 1)):
+        got = nf24_linear(*t, output_start=start, output_count=count)
+        assert torch.equal(got, full[:, start:start + count]), (start, count)

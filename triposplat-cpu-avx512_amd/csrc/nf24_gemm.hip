@@ -422,11 +422,7 @@ int launch_cfg(const GemmParams& p, hipStream_t stream, const QkvArgs& e = QkvAr
   const int64_t tiles = (int64_t)tiles_m * tiles_n;
   if (tiles <= 0 || tiles > 0x7fffffff) return kErrDims;
   xcd_blocking(tiles_m, tiles_n, C::BM, C::BN, p.K, a.xcd_pm, a.xcd_pn);
-  const bool vec = (reinterpret_cast<uintptr_t>(p.x) % 16 == 0) && (p.stride_x % 4 == 0) &&
-                   (p.K % 4 == 0) && (p.N % 2 == 0) && (p.n_start % 2 == 0) &&
-                   (p.n_count % 2 == 0) && (reinterpret_cast<uintptr_t>(p.code01) % 4 == 0) &&
-                   (reinterpret_cast<uintptr_t>(p.q2) % 2 == 0) &&
-                   vec_buffers_fit(p, C::BM, C::BK);
+  const bool vec = pair_loads_fit(p, C::BM, C::BK);
   // The scalar path's configuration covers the same tiles, possibly with
   // another K step or wave layout (and so another workgroup size).
   using S = typename ScalarPathCfg<C>::type;

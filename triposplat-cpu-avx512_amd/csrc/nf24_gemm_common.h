@@ -299,6 +299,15 @@ inline bool vec_buffers_fit(const GemmParams& p, int bm, int bk) {
          ((int64_t)(bm - 1) * p.stride_x + p.K + bk) * 4 < kLimit;
 }
 
+// Whether the fp32 MFMA tiles' vector loads (four x values, two columns of
+// codes) take the call.
+inline bool pair_loads_fit(const GemmParams& p, int bm, int bk) {
+  return (reinterpret_cast<uintptr_t>(p.x) % 16 == 0) && (p.stride_x % 4 == 0) && (p.K % 4 == 0) &&
+         (p.N % 2 == 0) && (p.n_start % 2 == 0) && (p.n_count % 2 == 0) &&
+         (reinterpret_cast<uintptr_t>(p.code01) % 4 == 0) && (reinterpret_cast<uintptr_t>(p.q2) % 2 == 0) &&
+         vec_buffers_fit(p, bm, bk);
+}
+
 // bf16-MFMA GEMM (nf24_gemm_bf16.hip) for p.precision kPrecisionBf16 /
 // kPrecisionBf16x3 and M > 32: epilogue kind epi (kEpi* / kEpilogue*), QKV
 // operands e, gate operands ep, token index of row 0 row0.

@@ -734,13 +734,25 @@ bool gemm_f16_vector(const GemmParams& p) {
          vec_buffers_fit(p, F16Large::BM, F16Large::BK);
 }
 
-// Operands the vector loads do not take (unaligned, odd strides or sizes)
-// make the element-wise loads the cost, where the fp32 tiles are the faster
-// (9000 x 998 x 1030 302 against 348 us, 4096 x 1002 x 3070 304 against 353),
-// so from 256 rows and columns on those calls stay with nf24_gemm.hip.  Below,
-// where either is a few tiles, the fp16 products serve every call, so that an
-// unaligned column range of a small call holds the bits of the whole call.
-bool gemm_f16_takes(const GemmParams& p) { return p.M < 256 || p.n_count < 256 || gemm_f16_vector(p); }
+// Calls that the vector loads do not take read element by element, and that is
+// then the cost.  The fp32 tiles serve those
+//   * whose weight they load in pairs of columns (N % 4 == 2): 33 to 255 rows of
+//     1024 x 1002 47 us against 58 to 64 here, 12294 x 1024 x 254 85 against
+//     115, 4096 x 4096 x 254 185 against 270;
+//   * of 256 rows and columns or more, where both read element by element (9000
+//     x 1030 x 998 302 against 348).
+// The fp16 products serve the other small ones (33 to 255 rows of 1030 x 1024
+// 84 to 94 us there, 58 here; 4096 x 1024 x 5 91 and 60): the weight decides
+// first, so that an unaligned column range of a small call holds the bits of
+// the whole call.
+bool gemm_f16_takes(const GemmParams& p) {
+  if (gemm_f16_vector(p)) return true;
+  GemmParams whole = p;
+  whole.n_start = 0;
+  whole.n_count = p.N;
+  if (!gemm_f16_vector(whole) && pair_loads_fit(whole, F16Large::BM, F16Large::BK)) return false;
+  return p.M < 256 || p.n_count < 256;
+}
 
 int launch_gemm_f16(const GemmParams& p, int epi, const QkvArgs& e, const GemmEpilogueParams& ep, int row0,
                     hipStream_t stream) {
