@@ -207,3 +207,30 @@ def test_ranges_of_any_alignment(oracle, cuda, hiplib, M, K, N):
     for start, count in ((0, 2), (2, 6), (5, 7), (4, 100), (N - 1, 1), (1, N - 1)):
         got = nf24_linear(*t, output_start=start, output_count=count)
         assert torch.equal(got, full[:, start:start + count]), (start, count)
+
+
+def test_capture_before_any_eager_call(oracle, cuda, hiplib):
+    """A row tail that only the fp16 tiles split off: a capture on a stream
+    without a workspace keeps it in the tiles."""
+    import torch
+    from tsplat.nf24 import nf24_linear
+
+    M, K, N = 6913, 1024, 1664
+    x, w, b = seeded_linear(3, M, K, N, w_scale=0.02)
+    c01, q2, s = oracle.quantize_nf24_i16(w)
+    t = [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (x, c01, q2, s, b)]
+    want = nf24_linear(*t)
+    out = torch.empty_like(want)
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=stream, capture_error_mode="relaxed"):
+        nf24_linear(*t, out=out)
+    for _ in range(3):
+        out.fill_(float("nan"))
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out[:-1], want[:-1])
+        rows = slice(M - 1, M)
+        _check(oracle, x[rows], c01, q2, s, b, out[rows].cpu().numpy())
+        assert torch.equal(nf24_linear(*t), want)
