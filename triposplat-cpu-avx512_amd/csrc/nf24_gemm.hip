@@ -728,6 +728,8 @@ int launch_epi_kind(const GemmParams& p, const GemmEpilogueParams& e, hipStream_
 }
 }  // namespace
 
+int nf24::fp32_tail_rows(int M, int n_count) { return tail_rows(M, n_count); }
+
 int nf24::launch_strict_tail(const GemmParams& p, int epi, const QkvArgs& e,
                              const GemmEpilogueParams& ep, int row0, hipStream_t stream) {
   GemmParams s = p;

@@ -762,7 +762,9 @@ int launch_gemm_f16(const GemmParams& p, int epi, const QkvArgs& e, const GemmEp
   if (!gemm_f16_vector(p)) return launch_cfg<F16Narrow, false>(a, epi, stream);
   // At most 32 rows past the last multiple of 256 run on the few-row kernels
   // when they would add a round of tiles (their workspace is the only thing
-  // that can fail, so they go first).
+  // that can fail, so they go first).  Without the workspace (a capture that
+  // would need it to grow) they stay in the tiles, except where the fp32 tiles
+  // split them off too: those calls fail, as they do in every mode.
   const int rem = p.M % 256;
   if (rem != 0 && rem <= 32 &&
       model_time(pick(p.M, p.n_count), p.M, p.n_count) >
@@ -772,8 +774,8 @@ int launch_gemm_f16(const GemmParams& p, int epi, const QkvArgs& e, const GemmEp
     if (p.out != nullptr) t.out = p.out + (int64_t)(p.M - rem) * p.stride_out;
     t.M = rem;
     const int st = launch_strict_tail(t, epi, e, ep, row0 + p.M - rem, stream);
-    if (st != kOk) return st;
-    a.M = p.M - rem;
+    if (st == kOk) a.M = p.M - rem;
+    else if (st != kErrWorkspace || fp32_tail_rows(p.M, p.n_count) != 0) return st;
   }
   switch (pick(a.M, p.n_count)) {
     case 0: return launch_cfg<F16Large, true>(a, epi, stream);
