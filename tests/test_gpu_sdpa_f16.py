@@ -128,3 +128,37 @@ def test_not_finite(cuda):
     assert np.all(np.isnan(got[0, 0, 4]))
     rest = np.setdiff1d(np.arange(66), [4])
     assert np.array_equal(got[0, 0][rest], base[0, 0][rest])
+
+
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("biased", [False, True])
+@pytest.mark.parametrize("Lq,Lk", [(40, 16384), (8200, 4096)])
+@pytest.mark.parametrize("bits", [26, 29, 31])
+def test_many_small_weights(cuda, Lq, Lk, biased, packed, bits):
+    """One key 2^(bits + 0.4) above all others, which are alike and whose values
+    share a mean: together they weigh Lk 2^-(bits + 0.4), and that has to reach
+    the result."""
+    import torch
+
+    H = 2 if Lq < 100 else 16
+    q, k, v = _qkv(bits, 1, H, Lq, Lk)
+    v = (1.0 + 0.05 * v).astype(np.float32)
+    v[:, :, 77] = 0.0
+    gap = np.float32((bits + 0.4) * math.log(2.0))
+    k[:] = 0.0
+    b = None
+    if biased:
+        b = np.full(Lk, -gap, np.float32)
+        b[77] = 0.0
+    else:
+        q[:] = 1.0
+        k[:, :, 77] = gap / 8.0
+    rows = np.arange(0, min(Lq, 64))
+    got = _run(torch, cuda, q, k, v, b, packed=packed)[:, :, rows]
+    exact = sdpa_f64(q[:, :, rows], k, v, b)
+    # exponents of up to 32 in log2 units, rounded twice, and fp32 sums over at
+    # most 512 blocks of 32 like keys: (2 * 32 + 512) * 2^-24 of the small weights;
+    # and a weight is held to 2^-36 of the largest (|v| < 1.3)
+    err = float(np.abs(got - exact).max())
+    rest = Lk * 2.0 ** -(bits + 0.4)
+    assert err <= 1.3 * (576 * 2.0 ** -24 * rest + Lk * 2.0 ** -36), err / rest

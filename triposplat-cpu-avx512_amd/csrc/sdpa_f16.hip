@@ -7,7 +7,7 @@
 // power-of-two scale and each product as three fp16 products with fp32
 // accumulation:
 //   q sq = qh + ql,  k sk = kh + kl,  S = (qh.kh + ql.kh + qh.kl) / (sq sk)
-//   2^4 p = ph + pl, v sv = vh + vl,  O = (ph vh + pl vh + ph vl) / (2^4 sv)
+//   2^11 p = ph + pl, v sv = vh + vl, O = (ph vh + pl vh + ph vl) / (2^11 sv)
 // A pair holds its value to one unit of fp32's last place down to 2^-24 of
 // the scale and to 2^-25 of the scale below that; the dropped low x low
 // product is below 2^-22 of the product (2^-24 rms).  sq is the query row's
@@ -22,7 +22,8 @@
 // Softmax in log2 units with a lazy reference: p = exp2(x - m + 4) for a
 // reference m that follows the running maximum only when that has moved by
 // more than 4, so p stays below 2^8 and most 32-key blocks rescale nothing;
-// the sums and the outputs share the factor.  Without a bias the exponent is
+// the sums and the outputs share the factor, which 2^7 more bring up to the
+// pairs' range.  Without a bias the exponent is
 // one FMA of the accumulator; with one as well, and a block that moves the
 // reference computes its scores again.
 //
@@ -75,6 +76,11 @@ constexpr int kWaitVmcnt0 = 0x0f70;  // s_waitcnt operand: vector-memory count 0
 constexpr float kPBase = 4.0f;
 constexpr float kSlack = 4.0f;
 constexpr float kStart = -3.0e38f;   // the reference before any key
+// p is taken up by 2^kPShift before it is split: below 2^15, and held to 2^-25,
+// 2^-36 of a weight at the reference (many small weights add up: 16384 of them,
+// each 2^-30 of one key's, were lost to the pairs, not to their sum).  After the
+// exponential, so that its argument stays small.
+constexpr int kPShift = 7;
 
 // Position of tile key k in a V^T row: bits 2 and 3 swapped.
 __device__ __forceinline__ int vt_pos(int k) { return (k & ~12) | ((k & 4) << 1) | ((k & 8) >> 1); }
@@ -537,7 +543,7 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_f16_kernel(SdpaArgs a, const
         float ls = 0.0f;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          s[r] = __builtin_amdgcn_exp2f(kBias ? s[r] : fmaf(s[r], ce, -re));
+          s[r] = __builtin_amdgcn_exp2f(kBias ? s[r] : fmaf(s[r], ce, -re)) * (float)(1 << kPShift);
           ls += s[r];
         }
         l_run += ls;
@@ -565,12 +571,14 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_f16_kernel(SdpaArgs a, const
     __syncthreads();
   }
 
+  // sums and outputs of weights of at most 1 (kPBase + kSlack + kPShift = 15),
+  // which overflow no sooner than the result
   const float unscale = inverse_pow2(sv);
 #pragma unroll
   for (int db = 0; db < 2; ++db)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) o[db][r] *= unscale;
-  store_rows<kBQ>(a, o, m_run, l_run);
+    for (int r = 0; r < 16; ++r) o[db][r] = o[db][r] * 0x1p-15f * unscale;
+  store_rows<kBQ>(a, o, m_run, l_run * 0x1p-15f);
 }
 
 template <int kLayout, bool kBias, int kWaves, bool kPre>
