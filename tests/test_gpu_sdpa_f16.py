@@ -162,3 +162,83 @@ def test_many_small_weights(cuda, Lq, Lk, biased, packed, bits):
     err = float(np.abs(got - exact).max())
     rest = Lk * 2.0 ** -(bits + 0.4)
     assert err <= 1.3 * (576 * 2.0 ** -24 * rest + Lk * 2.0 ** -36), err / rest
+
+
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("H,Lq,Lk", [(2, 70, 300), (2, 70, 1200), (16, 8200, 300)])
+@pytest.mark.parametrize("size", [1e4, 1e8, 1e12, 1e30, 1e36])
+@pytest.mark.parametrize("mask", [-math.inf, -1e30])
+def test_masked_keys_of_any_size(cuda, H, Lq, Lk, size, mask, packed):
+    """What a masked key holds, in k or in v, changes nothing (a finite mask: as
+    long as its scores stay below the others)."""
+    import torch
+
+    q, k, v = _qkv(int(math.log10(size)) + Lk, 1, H, Lq, Lk)
+    print(f"sdpa masked H={H} Lq={Lq} Lk={Lk} size={size} mask={mask} packed={packed}", flush=True)
+    cols = np.r_[0:3, 40:90, Lk - 50:Lk]
+    live = np.setdiff1d(np.arange(Lk), cols)
+    b = np.zeros(Lk, np.float32)
+    b[cols] = mask
+    rows = np.arange(0, 64)
+    exact = sdpa_f64(q[:, :, rows], k[:, :, live], v[:, :, live])
+    sign = np.sign(v[:, :, cols]).astype(np.float32)
+    v2 = v.copy()
+    v2[:, :, cols] = sign * np.float32(size)
+    got = _run(torch, cuda, q, k, v2, b, packed=packed)[:, :, rows]
+    assert stats(got, exact)["rel_rmse"] < 2e-6
+    if math.isinf(mask) or size < 1e29:  # (q k below the finite mask)
+        k2 = k.copy()
+        k2[:, :, cols] = sign * np.float32(size)
+        got = _run(torch, cuda, q, k2, v2, b, packed=packed)[:, :, rows]
+        assert stats(got, exact)["rel_rmse"] < 2e-6
+
+
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("H,Lq,Lk,bias", [(2, 70, 300, False), (2, 70, 1200, True), (16, 8200, 300, False),
+                                          (16, 8200, 300, True)])
+@pytest.mark.parametrize("dims", [[5], [0, 17, 63]])
+def test_outlier_dims(cuda, H, Lq, Lk, bias, dims, packed):
+    """Dims of v far larger than the rest cost the rest nothing; dims of k far
+    larger than the rest, where q is zero, cost the scores nothing."""
+    import torch
+
+    q, k, v = _qkv(5 + Lk, 1, H, Lq, Lk)
+    print(f"sdpa outlier dims H={H} Lq={Lq} Lk={Lk} bias={bias} dims={dims} packed={packed}", flush=True)
+    b = np.random.default_rng(1).uniform(-2, 0, Lk).astype(np.float32) if bias else None
+    rows = np.arange(0, 64)
+    keep = np.setdiff1d(np.arange(64), dims)
+    q[:, :, :, dims] = 0.0
+    exact = sdpa_f64(q[:, :, rows], k, v, b)
+    for size in (1e6, 1e12, 1e25):
+        v2, k2 = v.copy(), k.copy()
+        v2[:, :, :, dims] *= np.float32(size)
+        got = _run(torch, cuda, q, k, v2, b, packed=packed)[:, :, rows]
+        assert stats(got[..., keep], exact[..., keep])["rel_rmse"] < 2e-6, size
+        assert stats(got[..., dims], exact[..., dims] * size)["rel_rmse"] < 2e-6, size
+        k2[:, :, :, dims] *= np.float32(size)
+        got = _run(torch, cuda, q, k2, v, b, packed=packed)[:, :, rows]
+        assert stats(got, exact)["rel_rmse"] < 2e-6, size
+
+
+@pytest.mark.parametrize("Lq", [40, 8200])
+def test_tokens_of_any_size(cuda, Lq):
+    """Key tiles whose values of v differ by any power: each query's weight lies
+    on the keys of one tile, and its result has that tile's precision."""
+    import torch
+
+    H, Lk = (1, 320) if Lq < 100 else (16, 320)
+    q, k, v = _qkv(21, 1, H, Lq, Lk)
+    size = np.float32([1.0, 1e-25, 1e12, 3e-10, 1e30])
+    tile = np.repeat(np.arange(5), 64)
+    v = (v * size[tile][:, None]).astype(np.float32)
+    k = 0.01 * k
+    k[:, :, np.arange(Lk), tile] += 1.0
+    q[:] = 0.0
+    want = np.arange(Lq) % 5
+    q[:, :, np.arange(Lq), want] = 3000.0                 # 375 above the keys of the other tiles
+    got = _run(torch, cuda, q, k, v)
+    exact = sdpa_f64(q[:, :, :64], k, v)
+    for i in range(5):
+        r = np.nonzero(want[:64] == i)[0]
+        # scores of about 375, fp32's last place of which is 2^-16
+        assert stats(got[:, :, r] / size[i], exact[:, :, r] / size[i])["rel_rmse"] < 1e-4, i

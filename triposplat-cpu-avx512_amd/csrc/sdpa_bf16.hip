@@ -433,7 +433,7 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_bf16_kernel(SdpaArgs a, cons
     __syncthreads();
   }
 
-  store_rows<kBQ>(a, o, m_run, l_run);
+  store_rows<kBQ>(a, o, m_run, l_run, threadIdx.x);
 }
 
 template <int kLayout, bool kBias, int kTerms, int kWaves, bool kPre>

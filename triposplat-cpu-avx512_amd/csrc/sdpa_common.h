@@ -137,20 +137,31 @@ __device__ __forceinline__ TileWork tile_work(const SdpaArgs& a) {
   return w;
 }
 
+__device__ __forceinline__ void store4(float* dst, const floatx4& y, bool only_non_finite) {
+  if (only_non_finite) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (!(fabsf(y[e]) < INFINITY)) dst[e] = y[e];
+  } else {
+    *reinterpret_cast<floatx4*>(dst) = y;
+  }
+}
+
 // Final store of a wave's 32 queries: o[db][r] holds O^T[db*32 + 8*(r/4) +
 // 4*g + r%4][query] (the 32x32 MFMA accumulator layout), m_run / l_run the
 // lane's running max and partial sum.  Split parts write the unnormalised
 // rows and (max, sum) for the combine kernel.  The tile indices are
 // recomputed here from the launch state rather than kept live across the
-// key loop (fewer registers held through it).
+// key loop (fewer registers held through it).  only_non_finite: stores the
+// outputs that are infinite or NaN alone (over those another pass stored).
 template <int kBQ>
 __device__ __forceinline__ void store_rows(const SdpaArgs& a, const floatx16 (&o)[2], float m_run,
-                                           float l_run) {
+                                           float l_run, int tid, bool only_non_finite = false) {
   const TileWork w = tile_work(a);
   int bh, qb;
   tile_coords(a, w.tile, kBQ, bh, qb);
   const int b = bh / a.H, h = bh % a.H, part = w.part;
-  const int wave = threadIdx.x >> 6, g = (threadIdx.x >> 5) & 1, l32 = threadIdx.x & 31;
+  const int wave = tid >> 6, g = (tid >> 5) & 1, l32 = tid & 31;
   const int qrow = qb * kBQ + wave * 32 + l32;
   if (qrow >= a.Lq) return;  // lanes l and l ^ 32 share the query: both leave or neither
   const float lsum = pair_sum(l_run);
@@ -164,9 +175,9 @@ __device__ __forceinline__ void store_rows(const SdpaArgs& a, const floatx16 (&o
         floatx4 y;
 #pragma unroll
         for (int e = 0; e < 4; ++e) y[e] = o[db][4 * r4 + e];
-        *reinterpret_cast<floatx4*>(po + db * 32 + 8 * r4 + 4 * g) = y;
+        store4(po + db * 32 + 8 * r4 + 4 * g, y, only_non_finite);
       }
-    if (g == 0) {
+    if (g == 0 && !only_non_finite) {
       a.part_ml[2 * row] = m_run;
       a.part_ml[2 * row + 1] = lsum;
     }
@@ -182,7 +193,7 @@ __device__ __forceinline__ void store_rows(const SdpaArgs& a, const floatx16 (&o
       floatx4 y;
 #pragma unroll
       for (int e = 0; e < 4; ++e) y[e] = o[db][4 * r4 + e] * inv;
-      *reinterpret_cast<floatx4*>(dst + db * 32 + 8 * r4 + 4 * g) = y;
+      store4(dst + db * 32 + 8 * r4 + 4 * g, y, only_non_finite);
     }
 }
 

@@ -8,28 +8,34 @@
 // accumulation:
 //   q sq = qh + ql,  k sk = kh + kl,  S = (qh.kh + ql.kh + qh.kl) / (sq sk)
 //   2^11 p = ph + pl, v sv = vh + vl, O = (ph vh + pl vh + ph vl) / (2^11 sv)
-// A pair holds its value to one unit of fp32's last place down to 2^-24 of
-// the scale and to 2^-25 of the scale below that; the dropped low x low
-// product is below 2^-22 of the product (2^-24 rms).  sq is the query row's
-// own, sk and sv are the (b, h)'s: they bring the largest finite magnitude to
-// [2^14, 2^15), so what a score or an output loses to the scale is below
-// 2^-37 of |q| |k|max or |v|max.  Products of fp16 values are exact in fp32
-// and the matrix core rounds its accumulator twice per 16 products, so the
-// error against 64 bits is below the fp32 MFMA kernel's (16 heads, L = 16384:
-// 1.5e-6 against 2.3e-6 relative; L = 8194 with log(8194) on one key 2.2e-7,
-// as there).
+// A pair holds its value to one unit of fp32's last place down to 2^-2, and to
+// 2^-25 below that; the dropped low x low product is below 2^-22 of the product
+// (2^-24 rms).  sq is the query row's own, sk and sv are the key tile's: they
+// bring its largest magnitude to [2^14, 2^15) (v's to [2^11, 2^15)).  Products of
+// fp16 values are exact in fp32 and the matrix core rounds its accumulator twice
+// per 16 products, so the error against 64 bits is below the fp32 MFMA kernel's
+// (16 heads, L = 16384: 1.5e-6 against 2.3e-6 relative; L = 8194 with log(8194)
+// on one key 2.2e-7, as there).
+//
+// What the pairs do not serve.  Values far below their tile's largest lose
+// precision, and that matters where the large ones do not count: keys that a
+// bias removes, dims that q leaves out.  So every four neighbouring values of v
+// that are not all zero have to reach 2^-5 of the scale (2^-16 of the tile's
+// largest value at worst; they are then held to 2^-20), and where values of q or
+// k spread over more than 2^18 |q| |k| has to stay below 2^14, so that what a
+// score loses (64 dims of 2^-39 |q| |k|) stays below 2^-20.  A workgroup that
+// meets a tile which fails this, an infinity in q or k, or tiles of v more than
+// 2^64 apart, runs its queries and keys as fp32 products (sdpa_fp32.h) instead:
+// what another key or dim holds costs a result nothing that it would not cost
+// there.  (8194 keys with a bias, 50 of them masked and holding 1e30: 2166 us; the
+// fp32 tiles 2150.)
 //
 // Softmax in log2 units with a lazy reference: p = exp2(x - m + 4) for a
 // reference m that follows the running maximum only when that has moved by
 // more than 4, so p stays below 2^8 and most 32-key blocks rescale nothing;
 // the sums and the outputs share the factor, which 2^7 more bring up to the
-// pairs' range.  Without a bias the exponent is
-// one FMA of the accumulator; with one as well, and a block that moves the
-// reference computes its scores again.
-//
-// An infinity or NaN of k or v does not enter the scales and sits in the low
-// part alone (the high part is held to +-65504), where it meets qh or ph: the
-// score or output it makes is the one fp32 products would give.
+// pairs' range.  Without a bias the exponent is one FMA of the accumulator; with
+// one as well, and a block that moves the reference computes its scores again.
 //
 // Mapping, fragments and LDS image as in sdpa_bf16.hip: a wave owns 32
 // queries and computes S^T = K Q^T with v_mfma_f32_32x32x16_f16, each lane
@@ -42,16 +48,18 @@
 // otherwise each workgroup splits the tiles it reads.  Both place the same
 // values, so they give the same bits.
 //
-// Measured (16 heads) against the fp32 MFMA kernel: L = 16384 7.88 -> 2.75 ms
-// (400 TFLOP/s), 12294 4.57 -> 1.62 ms, 8194 with a key bias 2.14 -> 0.81 ms,
-// 4096 x 2048 280 -> 143 us, 577 52 -> 39 us.  What bounds it: the fp16 matrix
+// Measured (16 heads) against the fp32 MFMA kernel: L = 16384 7.89 -> 2.79 ms
+// (394 TFLOP/s), 8194 with a key bias 2.15 -> 0.82 ms, 4096 x 2048 282 -> 157 us,
+// 2 x 4096 x 4096 1022 -> 424 us, 577 52 -> 37 us, 2 x 1025 x 513 87 -> 50 us (a
+// scale per head instead, from a look at all of its keys: 2.80 ms, 0.82 ms, 159,
+// 429, 42 and 56 us).  What bounds it: the fp16 matrix
 // cores at the clock they hold, 1.2 PFLOP/s at L = 16384 where a plain 8192^3
 // fp16 library product reaches 1.11 (waves of 64 queries, which read half the
 // LDS fragments per product, 3.05 against 2.97 ms; wave priorities no change).
 // The 128-query tiles are split along the keys where CUs would idle
-// (plan_key_ranges): 300 x 9000 420 -> 102 us.
+// (plan_key_ranges): 300 x 9000 654 -> 88 us.
 
-#include "sdpa_common.h"
+#include "sdpa_fp32.h"
 
 namespace tsplat {
 namespace sdpa {
@@ -76,6 +84,16 @@ constexpr int kWaitVmcnt0 = 0x0f70;  // s_waitcnt operand: vector-memory count 0
 constexpr float kPBase = 4.0f;
 constexpr float kSlack = 4.0f;
 constexpr float kStart = -3.0e38f;   // the reference before any key
+// Largest |q| |k| (of a wave's queries, of a key tile) whose scores the pairs
+// serve: any, short of the scales' own range, where neither operand's values
+// spread over more than its pairs hold; elsewhere as long as 64 dims of 2^-39
+// |q| |k| stay below 2^-20 of a log2 unit.
+constexpr float kPairTop = 0x1p96f;
+constexpr int kEvRange = 1024;  // beyond any ev
+// How far apart the tiles' scales of v may be: outputs below 2^44 in the unit
+// of one tile stay in range in that of another.
+constexpr int kEvSpread = 64;
+constexpr float kWideTop = 0x1p14f;
 // p is taken up by 2^kPShift before it is split: below 2^15, and held to 2^-25,
 // 2^-36 of a weight at the reference (many small weights add up: 16384 of them,
 // each 2^-30 of one key's, were lost to the pairs, not to their sum).  After the
@@ -86,21 +104,17 @@ constexpr int kPShift = 7;
 __device__ __forceinline__ int vt_pos(int k) { return (k & ~12) | ((k & 4) << 1) | ((k & 8) >> 1); }
 
 // (hi, lo) of a and b: hi = fp16(v), lo = fp16(v - hi), the difference exact
-// in fp32.  kClamp: hi within fp16's finite range.
-template <bool kClamp>
+// in fp32.
 __device__ __forceinline__ void split2(float a, float b, unsigned& hi, unsigned& lo) {
-  const float ca = kClamp ? __builtin_amdgcn_fmed3f(a, -65504.0f, 65504.0f) : a;
-  const float cb = kClamp ? __builtin_amdgcn_fmed3f(b, -65504.0f, 65504.0f) : b;
-  const half2v h = __builtin_convertvector(floatx2{ca, cb}, half2v);
+  const half2v h = __builtin_convertvector(floatx2{a, b}, half2v);
   hi = __builtin_bit_cast(unsigned, h);
   lo = __builtin_bit_cast(unsigned, __builtin_convertvector(floatx2{a - (float)h[0], b - (float)h[1]}, half2v));
 }
 
-template <bool kClamp>
 __device__ __forceinline__ void split4(const floatx4& v, half4v& hi, half4v& lo) {
   unsigned h[2], l[2];
-  split2<kClamp>(v[0], v[1], h[0], l[0]);
-  split2<kClamp>(v[2], v[3], h[1], l[1]);
+  split2(v[0], v[1], h[0], l[0]);
+  split2(v[2], v[3], h[1], l[1]);
   hi = __builtin_bit_cast(half4v, uintx2{h[0], h[1]});
   lo = __builtin_bit_cast(half4v, uintx2{l[0], l[1]});
 }
@@ -109,20 +123,19 @@ __device__ __forceinline__ void split4(const floatx4& v, half4v& hi, half4v& lo)
 __device__ __forceinline__ void split8(const floatx16& s, int c, half8& hi, half8& lo) {
   unsigned h[4], l[4];
 #pragma unroll
-  for (int e = 0; e < 4; ++e) split2<false>(s[8 * c + 2 * e], s[8 * c + 2 * e + 1], h[e], l[e]);
+  for (int e = 0; e < 4; ++e) split2(s[8 * c + 2 * e], s[8 * c + 2 * e + 1], h[e], l[e]);
   hi = __builtin_bit_cast(half8, uintx4{h[0], h[1], h[2], h[3]});
   lo = __builtin_bit_cast(half8, uintx4{l[0], l[1], l[2], l[3]});
 }
 
-// Power of two that brings a magnitude (as bits) to [2^14, 2^15), with a
-// normal reciprocal; 1 for zero.
-__device__ __forceinline__ float scale_for(uint32_t mx_bits) {
-  const int field = 268 - (int)(mx_bits >> 23);
-  return mx_bits == 0 ? 1.0f : __uint_as_float((uint32_t)min(max(field, 1), 253) << 23);
+// Exponent of the power of two that brings a magnitude (as bits) to [2^14,
+// 2^15), of a normal number and with a normal reciprocal; 0 for zero, infinity
+// and NaN.
+__device__ __forceinline__ int scale_exp(uint32_t mx_bits) {
+  const int e = 14 + 127 - (int)(mx_bits >> 23);
+  return mx_bits == 0 || mx_bits >= 0x7f800000u ? 0 : min(e, 126);
 }
-__device__ __forceinline__ float inverse_pow2(float s) {
-  return __uint_as_float((254u << 23) - __float_as_uint(s));
-}
+__device__ __forceinline__ float pow2(int e) { return __uint_as_float((uint32_t)(e + 127) << 23); }
 
 // Bits of |x|, 0 for an infinity or NaN.
 __device__ __forceinline__ uint32_t finite_bits(float x) {
@@ -130,72 +143,123 @@ __device__ __forceinline__ uint32_t finite_bits(float x) {
   return u < 0x7f800000u ? u : 0u;
 }
 
-// Largest finite magnitudes of k and v (as bits) over units first, first +
-// step, ... below `end` of one (b, h); a unit is 4 consecutive floats.
-template <int kLayout>
-__device__ __forceinline__ void kv_max(const SdpaArgs& a, const float* kbase, const float* vbase, int64_t first,
-                                       int64_t end, int step, uint32_t& km, uint32_t& vm) {
-  for (int64_t u = first; u < end; u += step) {
-    const floatx4 kx = *reinterpret_cast<const floatx4*>(kbase + 4 * u);
-    const floatx4 vx = *reinterpret_cast<const floatx4*>(vbase + 4 * u);
-    // key-contiguous rows: keys past Lk are not part of the operand
-    const int key = kLayout == 1 ? (int)(u % (a.Lkp / 4)) * 4 : 0;
+// Largest magnitude of four values (an infinity's is infinite, a NaN's none).
+__device__ __forceinline__ uint32_t max4(const floatx4& v) {
+  return __float_as_uint(fmaxf(fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fabsf(v[2])), fabsf(v[3])));
+}
+
+// Magnitudes of one K/V tile (as bits): the largest of k and of v, and (negated,
+// so that all four are maxima and 0 stands for none) the smallest among the
+// largest of each staging unit of four that is not all zero.
+struct TileMax {
+  uint32_t kmax, vmax, klow, vlow;
+};
+__device__ __forceinline__ void merge(TileMax& m, const TileMax& o) {
+  m.kmax = max(m.kmax, o.kmax);
+  m.vmax = max(m.vmax, o.vmax);
+  m.klow = max(m.klow, o.klow);
+  m.vlow = max(m.vlow, o.vlow);
+}
+template <int kLoads>
+__device__ __forceinline__ TileMax unit_max(const floatx4 (&kr)[kLoads], const floatx4 (&vr)[kLoads]) {
+  TileMax m = {0, 0, 0, 0};
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const bool in = kLayout == 0 || key + e < a.Lk;
-      km = max(km, in ? finite_bits(kx[e]) : 0u);
-      vm = max(vm, in ? finite_bits(vx[e]) : 0u);
-    }
+  for (int j = 0; j < kLoads; ++j) {
+    const uint32_t k = max4(kr[j]), v = max4(vr[j]);
+    merge(m, TileMax{k, v, 0u - k, 0u - v});
   }
+  return m;
 }
-template <int kLayout>
-__device__ __forceinline__ int64_t kv_units(const SdpaArgs& a) {
-  return kLayout == 1 ? (int64_t)kD * a.Lkp / 4 : (int64_t)a.Lk * kD / 4;
+template <int kCtrl>
+__device__ __forceinline__ TileMax dpp(const TileMax& m) {
+  return TileMax{(uint32_t)__builtin_amdgcn_mov_dpp((int)m.kmax, kCtrl, 0xf, 0xf, true),
+                 (uint32_t)__builtin_amdgcn_mov_dpp((int)m.vmax, kCtrl, 0xf, 0xf, true),
+                 (uint32_t)__builtin_amdgcn_mov_dpp((int)m.klow, kCtrl, 0xf, 0xf, true),
+                 (uint32_t)__builtin_amdgcn_mov_dpp((int)m.vlow, kCtrl, 0xf, 0xf, true)};
 }
+// Over the 16 lanes of a row: lane ^ 1, lane ^ 2, halves mirrored, row mirrored.
+__device__ __forceinline__ void row_max(TileMax& m) {
+  merge(m, dpp<0xb1>(m));
+  merge(m, dpp<0x4e>(m));
+  merge(m, dpp<0x141>(m));
+  merge(m, dpp<0x140>(m));
+}
+
+// The maxima over the workgroup, uniform, with a barrier in between; red is
+// written again no sooner than another barrier later.
+template <int kWaves>
+__device__ __forceinline__ TileMax reduce_max(TileMax m, uintx4 (&red)[kWaves * 4]) {
+  const int tid = threadIdx.x;
+  row_max(m);
+  if (tid % 16 == 0) red[tid / 16] = uintx4{m.kmax, m.vmax, m.klow, m.vlow};
+  __syncthreads();
+  const uintx4 u = red[tid % (kWaves * 4)];
+  m = TileMax{u[0], u[1], u[2], u[3]};
+  row_max(m);
+  if constexpr (kWaves > 4) {
+    static_assert(kWaves == 16, "one row, or a wave, of partial maxima");
+#pragma unroll
+    for (int d = 16; d < 64; d <<= 1)
+      merge(m, TileMax{(uint32_t)__shfl_xor((int)m.kmax, d), (uint32_t)__shfl_xor((int)m.vmax, d),
+                       (uint32_t)__shfl_xor((int)m.klow, d), (uint32_t)__shfl_xor((int)m.vlow, d)});
+  }
+  return TileMax{(uint32_t)__builtin_amdgcn_readfirstlane(m.kmax), (uint32_t)__builtin_amdgcn_readfirstlane(m.vmax),
+                 (uint32_t)__builtin_amdgcn_readfirstlane(m.klow), (uint32_t)__builtin_amdgcn_readfirstlane(m.vlow)};
+}
+
+// A tile's scales, uniform over the workgroup: k * 2^ek and v * 2^ev bring the
+// largest finite magnitude to [2^14, 2^15) and, ev a multiple of 4 (so that tiles
+// of like values share it and the outputs keep their unit), to [2^11, 2^15).
+struct TileInfo {
+  int ek, ev;
+  uint32_t flags;
+  float kmax;
+};
+constexpr uint32_t kKWide = 1;  // some unit of k is below 2^-4 of its scale
+constexpr uint32_t kVZero = 2;  // v has no finite value but zero
+constexpr uint32_t kVInf = 4;   // an infinity in v: zero in the planes
+constexpr uint32_t kFp32 = 8;   // the pairs do not serve: an infinity in k, or a unit
+                                // of v below 2^-5 of its scale, or v of 2^100 and more
+template <int kWaves, int kLoads>
+__device__ __forceinline__ TileInfo tile_info(const floatx4 (&kr)[kLoads], const floatx4 (&vr)[kLoads],
+                                              uintx4 (&red)[kWaves * 4]) {
+  TileMax m = reduce_max<kWaves>(unit_max(kr, vr), red);
+  TileInfo t;
+  t.flags = 0;
+  if (m.vmax >= 0x7f800000u) {  // (uniform, rare) the same of v's finite values
+    t.flags = kVInf;
+    TileMax f = {0, 0, 0, 0};
+#pragma unroll
+    for (int j = 0; j < kLoads; ++j) {
+      uint32_t v = 0;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v = max(v, finite_bits(vr[j][e]));
+      merge(f, TileMax{0, v, 0, 0u - v});
+    }
+    __syncthreads();
+    f = reduce_max<kWaves>(f, red);
+    m.vmax = f.vmax;
+    m.vlow = f.vlow;
+  }
+  t.ek = scale_exp(m.kmax);
+  t.ev = scale_exp(m.vmax) & ~3;
+  t.kmax = __uint_as_float(m.kmax);
+  if (m.vmax == 0) t.flags |= kVZero;
+  if (m.klow != 0 && __uint_as_float(0u - m.klow) * pow2(t.ek) < 0x1p-4f) t.flags |= kKWide;
+  if (m.kmax >= 0x7f800000u || __uint_as_float(m.vmax) >= 0x1p100f ||
+      (m.vlow != 0 && __uint_as_float(0u - m.vlow) * pow2(t.ev) < 0x1p-5f))
+    t.flags |= kFp32;
+  return t;
+}
+// Whether the pairs serve a tile for queries of at most qmax, whose own spread
+// allows |q| |k| up to q_top.
+__device__ __forceinline__ bool pairs_serve(uint32_t flags, float kmax, float qmax, float q_top) {
+  return (flags & kFp32) == 0 && qmax * kmax <= ((flags & kKWide) != 0 ? fminf(q_top, kWideTop) : q_top);
+}
+
 template <int kLayout>
 __device__ __forceinline__ int64_t head_stride(const SdpaArgs& a) {
   return kLayout == 1 ? (int64_t)kD * a.Lkp : (int64_t)a.Lk * kD;
-}
-
-__device__ __forceinline__ uint32_t wave_max(uint32_t x) {
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) x = max(x, (uint32_t)__shfl_xor((int)x, d));
-  return x;
-}
-
-// Magnitudes of k and v over one of the kMaxParts parts of a (b, h)'s keys:
-// maxes[bh][part] = (k, v).
-constexpr int kMaxParts = 16;
-constexpr int kMaxThreads = 256;
-template <int kLayout>
-__global__ __launch_bounds__(kMaxThreads) void sdpa_f16_max_kernel(SdpaArgs a, uint2* maxes) {
-  __shared__ uint32_t red[2][kMaxThreads / 64];
-  const int bh = blockIdx.x / kMaxParts, part = blockIdx.x % kMaxParts;
-  const int64_t units = kv_units<kLayout>(a), per = (units + kMaxParts - 1) / kMaxParts;
-  uint32_t km = 0, vm = 0;
-  kv_max<kLayout>(a, a.k + bh * head_stride<kLayout>(a), a.v + bh * head_stride<kLayout>(a),
-                  part * per + threadIdx.x, min(units, (part + 1) * per), kMaxThreads, km, vm);
-  km = wave_max(km);
-  vm = wave_max(vm);
-  if (threadIdx.x % 64 == 0) {
-    red[0][threadIdx.x / 64] = km;
-    red[1][threadIdx.x / 64] = vm;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int i = 1; i < kMaxThreads / 64; ++i) {
-      km = max(km, red[0][i]);
-      vm = max(vm, red[1][i]);
-    }
-    maxes[blockIdx.x] = uint2{km, vm};
-  }
-}
-
-// sk and sv of a (b, h) from its parts.
-__device__ __forceinline__ void head_scales(const uint2* maxes, int bh, float& sk, float& sv) {
-  const uint2 m = maxes[(int64_t)bh * kMaxParts + threadIdx.x % kMaxParts];
-  sk = scale_for(wave_max(m.x));
-  sv = scale_for(wave_max(m.y));
 }
 
 // LDS image of one K/V tile: fp16 planes of kPlaneElems elements, 0 = K hi,
@@ -225,18 +289,24 @@ __device__ __forceinline__ void fetch_kv(const SdpaArgs& a, const float* kbase, 
 // Scales and splits the fetched units and places them in the planes: K as
 // key rows, V transposed to dim rows with its keys at vt_pos.
 template <int kLayout, int kThreads, int kLoads>
-__device__ __forceinline__ void place_kv(int tid, float sk, float sv, const floatx4 (&kr)[kLoads],
+__device__ __forceinline__ void place_kv(int tid, const TileInfo& t, const floatx4 (&kr)[kLoads],
                                          const floatx4 (&vr)[kLoads], _Float16* planes) {
   _Float16* khi = planes;
   _Float16* vhi = planes + kPlaneElems;
   _Float16* klo = planes + 2 * kPlaneElems;
   _Float16* vlo = planes + 3 * kPlaneElems;
+  const float sk = pow2(t.ek), sv = pow2(t.ev);
 #pragma unroll
   for (int j = 0; j < kLoads; ++j) {
     const int idx = tid + j * kThreads;
     half4v kh, kl, vh, vl;
-    split4<true>(kr[j] * sk, kh, kl);
-    split4<true>(vr[j] * sv, vh, vl);
+    split4(kr[j] * sk, kh, kl);
+    floatx4 v = vr[j] * sv;
+    if (t.flags & kVInf) {  // (uniform)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = fabsf(v[e]) < INFINITY ? v[e] : 0.0f;
+    }
+    split4(v, vh, vl);
     const int row = idx / (kD / 4), c = idx % (kD / 4);
     if constexpr (kLayout == 0) {
       // key row, dims 4c..4c+3
@@ -262,26 +332,27 @@ __device__ __forceinline__ void place_kv(int tid, float sk, float sv, const floa
 }
 
 // Global image of the staged tiles: per (b*H + h, tile of 64 keys), the LDS
-// planes without their row padding, then with a key bias the tile's 64 bias
-// values in log2 units (zero past Lk).
+// planes without their row padding, the tile's TileInfo, then with a key bias
+// its 64 bias values in log2 units (zero past Lk).
+constexpr int kPlaneBytes = kPlanes * kTileKeys * kTileKeys * 2;
+constexpr int kInfoBytes = 16;
 template <bool kBias>
-constexpr int kImageTileBytes = kPlanes * kTileKeys * kTileKeys * 2 + (kBias ? kTileKeys * 4 : 0);
+constexpr int kImageTileBytes = kPlaneBytes + kInfoBytes + (kBias ? kTileKeys * 4 : 0);
 constexpr int kPreThreads = 256;
 
 template <int kLayout, bool kBias>
-__global__ __launch_bounds__(kPreThreads) void sdpa_f16_presplit_kernel(SdpaArgs a, const uint2* maxes, uintx4* out,
-                                                                        int ntiles) {
+__global__ __launch_bounds__(kPreThreads) void sdpa_f16_presplit_kernel(SdpaArgs a, uintx4* out, int ntiles) {
   constexpr int kLoads = kTileKeys * kD / 4 / kPreThreads;
   constexpr int kUnits = kPlanes * kTileKeys * kTileKeys / 8;  // 16-byte units of the planes
   __shared__ __attribute__((aligned(16))) _Float16 lds[kPlanes * kPlaneElems];
+  __shared__ uintx4 red[kPreThreads / 16];
   const int tid = threadIdx.x;
   const int bh = blockIdx.x / ntiles, tile = blockIdx.x % ntiles;
   const int64_t head = head_stride<kLayout>(a);
   floatx4 kr[kLoads], vr[kLoads];
   fetch_kv<kLayout, kPreThreads, kLoads>(a, a.k + bh * head, a.v + bh * head, tid, tile * kTileKeys, kr, vr);
-  float sk, sv;
-  head_scales(maxes, bh, sk, sv);
-  place_kv<kLayout, kPreThreads, kLoads>(tid, sk, sv, kr, vr, lds);
+  const TileInfo info = tile_info<kPreThreads / 64>(kr, vr, red);
+  place_kv<kLayout, kPreThreads, kLoads>(tid, info, kr, vr, lds);
   __syncthreads();
   uintx4* dst = out + (int64_t)blockIdx.x * (kImageTileBytes<kBias> / 16);
 #pragma unroll
@@ -290,20 +361,27 @@ __global__ __launch_bounds__(kPreThreads) void sdpa_f16_presplit_kernel(SdpaArgs
     const int p = u / (kUnits / kPlanes), r = (u / 8) % kTileKeys, ch = u % 8;
     dst[u] = *reinterpret_cast<const uintx4*>(&lds[p * kPlaneElems + r * kRowElems + 8 * ch]);
   }
+  if (tid == 0)
+    dst[kUnits] = uintx4{(unsigned)info.ek, (unsigned)info.ev, info.flags, __float_as_uint(info.kmax)};
   if (kBias && tid < kTileKeys) {
     const int key = tile * kTileKeys + tid;
     const float* brow = a.bias + (int64_t)(bh % a.H) * a.bias_head_stride;
-    reinterpret_cast<float*>(dst + kUnits)[tid] = key < a.Lk ? brow[key] * kLog2e : 0.0f;
+    reinterpret_cast<float*>(dst + kUnits + 1)[tid] = key < a.Lk ? brow[key] * kLog2e : 0.0f;
   }
 }
 
 // kLayout: 0 = k and v [B, H, Lk, 64]; 1 = both key-contiguous [B, H, 64,
 // Lkp].  kWaves waves of 32 queries share each tile of 64 keys, taken in two
-// 32-key blocks.  kPre: the tiles come from the presplit image `pre` (kLayout
-// is then unused).  maxes: sdpa_f16_max_kernel's result, or null, and the
-// workgroup looks through its (b, h)'s k and v itself.
+// 32-key blocks.  kPre: the tiles come from the presplit image `pre`.
+//
+// A workgroup that meets a tile the pairs do not serve (pairs_serve, or values
+// of v too far apart for one unit of the outputs) drops what it has and runs
+// its queries and keys as fp32 products instead (sdpa_fp32.h); with the image it
+// looks first.  An infinity in v changes only its own dims: their outputs, and
+// no others, come from such a pass at the end.
 template <int kLayout, bool kBias, int kWaves, bool kPre>
-__global__ __launch_bounds__(kWaves * 64) void sdpa_f16_kernel(SdpaArgs a, const uint2* maxes, const uintx4* pre) {
+__global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(kWaves == 4 ? 2 : 4)))
+void sdpa_f16_kernel(SdpaArgs a, const uintx4* pre) {
   constexpr int kThreads = kWaves * 64;
   constexpr int kBQ = kWaves * 32;
   constexpr int kUnits = kTileKeys * kD / 4;  // float4 of K (and of V) per tile
@@ -312,8 +390,13 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_f16_kernel(SdpaArgs a, const
   constexpr int kPLoads = kPre ? kPUnits / kThreads : 1;
   static_assert(kPre ? kPLoads * kThreads == kPUnits : kLoads * kThreads == kUnits, "tile split");
   static_assert(kThreads >= kTileKeys, "bias row load");
-  __shared__ __attribute__((aligned(16))) _Float16 kvl[2][kPlanes * kPlaneElems];
+  __shared__ union {
+    __attribute__((aligned(16))) _Float16 planes[2][kPlanes * kPlaneElems];
+    Fp32Lds<kLayout, kTileKeys> fp32;
+  } lds;
   __shared__ __attribute__((aligned(16))) float bbuf[2][kTileKeys];
+  __shared__ uintx4 red[kWaves * 4];
+  auto& kvl = lds.planes;
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -330,62 +413,48 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_f16_kernel(SdpaArgs a, const
   const int qrow = qb * kBQ + wave * 32 + l32;
   const bool q_ok = qrow < a.Lq;
 
-  const float* kbase = a.k + (int64_t)bh * head_stride<kLayout>(a);
-  const float* vbase = a.v + (int64_t)bh * head_stride<kLayout>(a);
+  const float* kbase = a.k + bh * head_stride<kLayout>(a);
+  const float* vbase = a.v + bh * head_stride<kLayout>(a);
   const float* brow = kBias ? a.bias + (int64_t)h * a.bias_head_stride : nullptr;
   constexpr int kTileBytes = kImageTileBytes<kBias>;
   const char* pbase = kPre ? reinterpret_cast<const char*>(pre) +
                                  (int64_t)bh * ((a.Lk + kTileKeys - 1) / kTileKeys) * kTileBytes
                            : nullptr;
 
-  float sk, sv;
-  if (kPre || maxes != nullptr) {
-    head_scales(maxes, bh, sk, sv);
-  } else {
-    uint32_t km = 0, vm = 0;
-    kv_max<kLayout>(a, kbase, vbase, tid, kv_units<kLayout>(a), kThreads, km, vm);
-    km = wave_max(km);
-    vm = wave_max(vm);
-    uint32_t* red = reinterpret_cast<uint32_t*>(&kvl[0][0]);
-    if (lane == 0) {
-      red[2 * wave] = km;
-      red[2 * wave + 1] = vm;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < kWaves; ++i) {
-      km = max(km, red[2 * i]);
-      vm = max(vm, red[2 * i + 1]);
-    }
-    __syncthreads();
-    sk = scale_for(km);
-    sv = scale_for(vm);
-  }
-  sk = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(sk)));
-  sv = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(sv)));
-
   // Q slices in registers: dims 16c + 8g + i of the query under its own scale.
   half8 qh[4], ql[4];
-  float c1;  // log2 units per unit of the score accumulator
+  int eq;  // exponent of the query's scale
+  // The pairs serve a tile's scores where qmax, the workgroup's largest |q|, times
+  // the tile's largest |k| is at most q_top.
+  float qmax, q_top;
   {
     const float* qp = a.q + ((int64_t)bh * a.Lq + (q_ok ? qrow : 0)) * kD + 8 * g;
     floatx4 x[8];
-    uint32_t mx = 0;
+    uint32_t mx = 0, low = 0;
+    bool inf = false;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       x[i] = q_ok ? *reinterpret_cast<const floatx4*>(qp + 16 * (i / 2) + 4 * (i % 2)) : floatx4{0, 0, 0, 0};
+      uint32_t m = max4(x[i]);
+      inf |= m >= 0x7f800000u;
+      low = max(low, 0u - m);
 #pragma unroll
       for (int e = 0; e < 4; ++e) mx = max(mx, finite_bits(x[i][e]));
     }
     mx = __float_as_uint(pair_max(__uint_as_float(mx)));
-    const float sq = scale_for(mx);
-    // kept positive and finite, so that a masked score stays -inf
-    c1 = __builtin_amdgcn_fmed3f(0.125f * kLog2e * inverse_pow2(sq) * inverse_pow2(sk), 0x1p-126f, 0x1p127f);
+    eq = scale_exp(mx);
+    // (4 neighbouring dims of a query below 2^-4 of its scale)
+    const bool wide = low != 0 && __uint_as_float(0u - low) * pow2(eq) < 0x1p-4f;
+    TileMax m = {mx, 0, wide ? 1u : 0u, inf ? 1u : 0u};
+    m = reduce_max<kWaves>(m, red);
+    qmax = __uint_as_float(m.kmax);
+    q_top = m.vlow != 0 ? -1.0f : m.klow != 0 ? kWideTop : kPairTop;
+    __syncthreads();
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
       half4v hi[2], lo[2];
-      split4<false>(x[2 * c] * sq, hi[0], lo[0]);
-      split4<false>(x[2 * c + 1] * sq, hi[1], lo[1]);
+      split4(x[2 * c] * pow2(eq), hi[0], lo[0]);
+      split4(x[2 * c + 1] * pow2(eq), hi[1], lo[1]);
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         qh[c][e] = hi[e / 4][e % 4];
@@ -411,7 +480,7 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_f16_kernel(SdpaArgs a, const
 #pragma unroll
       for (int j = 0; j < kPLoads; ++j) pr[j] = reinterpret_cast<const uintx4*>(src)[tid + j * kThreads];
       if (kBias && __builtin_amdgcn_readfirstlane(wave) == kWaves - 1)
-        __builtin_amdgcn_global_load_lds(src + kPUnits * 16 + lane * 4,
+        __builtin_amdgcn_global_load_lds(src + kPUnits * 16 + kInfoBytes + lane * 4,
                                          (__attribute__((address_space(3))) void*)(&bbuf[buf][0]), 4, 0, 0);
     } else {
       fetch_kv<kLayout, kThreads, kLoads>(a, kbase, vbase, tid_s, key0, kr, vr);
@@ -421,7 +490,8 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_f16_kernel(SdpaArgs a, const
       }
     }
   };
-  auto store = [&](int buf) {
+  TileInfo info;  // of the tile placed last
+  auto store = [&](int key0, int buf) {
     int tid_s = tid;
     if constexpr (kWaves == 16 && !kPre) asm volatile("" : "+v"(tid_s));
     if constexpr (kPre) {
@@ -432,9 +502,13 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_f16_kernel(SdpaArgs a, const
         *reinterpret_cast<uintx4*>(&kvl[buf][p * kPlaneElems + r * kRowElems + 8 * ch]) = pr[j];
       }
       if constexpr (kBias) __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
+      const auto* ip = reinterpret_cast<const __attribute__((address_space(4))) unsigned*>(
+          reinterpret_cast<uintptr_t>(pbase + (int64_t)(key0 / kTileKeys) * kTileBytes + kPlaneBytes));
+      info = TileInfo{(int)ip[0], (int)ip[1], ip[2], __uint_as_float(ip[3])};
     } else {
-      place_kv<kLayout, kThreads, kLoads>(tid_s, sk, sv, kr, vr, kvl[buf]);
-      if (kBias && tid < kTileKeys) bbuf[buf][tid] = br;
+      info = tile_info<kWaves>(kr, vr, red);
+      place_kv<kLayout, kThreads, kLoads>(tid_s, info, kr, vr, kvl[buf]);
+      if (kBias && tid < kTileKeys) bbuf[buf][tid_s] = br;
     }
   };
 
@@ -448,13 +522,48 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_f16_kernel(SdpaArgs a, const
   // are then differences of rounded scores, 0 at the maximum
   bool huge = false;
   float l_run = 0.0f;
+  int ev = 0;  // the outputs' unit: 2^-ev
 
+  // (all uniform over the workgroup)
   const int ntiles = (w.k_end - w.k_begin + kTileKeys - 1) / kTileKeys;
-  load(w.k_begin, 0);
-  store(0);
-  __syncthreads();
+  int served = 1, v_inf = 0;
+  int ev_min = kEvRange, ev_max = -kEvRange;
+  if constexpr (kPre) {
+    bool bad = false, inf = false;
+    uint32_t hi = 0, lo = 0;
+    for (int i = tid; i < ntiles; i += kThreads) {
+      const uintx4 u = *reinterpret_cast<const uintx4*>(pbase + (int64_t)(w.k_begin / kTileKeys + i) * kTileBytes +
+                                                        kPlaneBytes);
+      bad |= !pairs_serve(u[2], __uint_as_float(u[3]), qmax, q_top);
+      inf |= (u[2] & kVInf) != 0;
+      if ((u[2] & kVZero) == 0) {
+        hi = max(hi, (uint32_t)(kEvRange + (int)u[1]));
+        lo = max(lo, (uint32_t)(kEvRange - (int)u[1]));
+      }
+    }
+    const TileMax m = reduce_max<kWaves>(TileMax{bad, inf, hi, lo}, red);
+    served = m.kmax == 0 && (int)(m.klow + m.vlow) <= 2 * kEvRange + kEvSpread ? 1 : 0;
+    v_inf = (int)m.vmax;
+  }
+  // Whether the tile placed last is one to go on with.
+  auto take = [&] {
+    v_inf |= (int)(info.flags & kVInf);
+    if ((info.flags & kVZero) == 0) {
+      ev_min = min(ev_min, info.ev);
+      ev_max = max(ev_max, info.ev);
+    }
+    served = pairs_serve(info.flags, info.kmax, qmax, q_top) && ev_max - ev_min <= kEvSpread ? 1 : 0;
+    return served != 0;
+  };
 
-  for (int t = 0; t < ntiles; ++t) {
+  if (served != 0) {
+    load(w.k_begin, 0);
+    store(w.k_begin, 0);
+    if (!kPre) (void)take();
+    __syncthreads();
+  }
+
+  for (int t = 0; served != 0 && t < ntiles; ++t) {
     const int buf = t & 1;
     const int key0 = w.k_begin + t * kTileKeys;
     if (t + 1 < ntiles) load(key0 + kTileKeys, buf ^ 1);
@@ -465,6 +574,17 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_f16_kernel(SdpaArgs a, const
     const bool tail = key0 + kTileKeys > a.Lk;
 
     if (wave_live) {
+      // log2 units per unit of the score accumulator, kept positive and finite,
+      // so that a masked score stays -inf
+      const float c1 =
+          __builtin_amdgcn_fmed3f(__builtin_amdgcn_ldexpf(0.125f * kLog2e, -eq - info.ek), 0x1p-126f, 0x1p127f);
+      if (info.ev != ev && (info.flags & kVZero) == 0) {
+#pragma unroll
+        for (int db = 0; db < 2; ++db)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) o[db][r] = __builtin_amdgcn_ldexpf(o[db][r], info.ev - ev);
+        ev = info.ev;
+      }
       // The 16-wave kernels have 128 registers: with a bias, or tiles split
       // here, the blocks and their phases are kept apart (one block in flight,
       // no instruction moved between scores, softmax and P V), or they spill.
@@ -567,25 +687,36 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_f16_kernel(SdpaArgs a, const
       }
     }  // wave_live
 
-    if (t + 1 < ntiles) store(buf ^ 1);
+    if (t + 1 < ntiles) {
+      store(key0 + kTileKeys, buf ^ 1);
+      if (!kPre && !take()) break;
+    }
     __syncthreads();
   }
 
-  // sums and outputs of weights of at most 1 (kPBase + kSlack + kPShift = 15),
-  // which overflow no sooner than the result
-  const float unscale = inverse_pow2(sv);
+  // (nothing of the query tile's coordinates is kept over the key tiles)
+  SdpaArgs e = a;
+  int tid_e = tid;
+  asm volatile("" : "+s"(e.Lq), "+s"(e.H), "+v"(tid_e));
+  tid_e &= kThreads - 1;  // (its range)
+  if (served != 0) {
+    // the outputs of weights exp2(x - m_run), as the fp32 tiles' partial rows
 #pragma unroll
-  for (int db = 0; db < 2; ++db)
+    for (int db = 0; db < 2; ++db)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) o[db][r] = o[db][r] * 0x1p-15f * unscale;
-  store_rows<kBQ>(a, o, m_run, l_run * 0x1p-15f);
+      for (int r = 0; r < 16; ++r) o[db][r] = __builtin_amdgcn_ldexpf(o[db][r], -(int)kPBase - kPShift - ev);
+    store_rows<kBQ>(e, o, m_run, l_run * 0x1p-11f, tid_e);
+    if (v_inf == 0) return;
+  }
+  __syncthreads();
+  sdpa_fp32_tile<kLayout, kBias, kWaves, kTileKeys, true>(e, lds.fp32.k, lds.fp32.v, bbuf, tid_e, served != 0);
 }
 
 template <int kLayout, bool kBias, int kWaves, bool kPre>
-int launch_shape(const SdpaParams& p, hipStream_t stream, const TilePlan& pl, const uint2* maxes, const uintx4* pre) {
+int launch_shape(const SdpaParams& p, hipStream_t stream, const TilePlan& pl, const uintx4* pre) {
   return launch_plan(make_args(p), p, pl, kWaves * 32, stream, [&](dim3 grid, const SdpaArgs& a) {
     hipLaunchKernelGGL((sdpa_f16_kernel<kLayout, kBias, kWaves, kPre>), grid, dim3(kWaves * 64), 0, stream, a,
-                       maxes, pre);
+                       pre);
   });
 }
 
@@ -593,14 +724,16 @@ int launch_shape(const SdpaParams& p, hipStream_t stream, const TilePlan& pl, co
 // key and head, as much as the fp32 K and V).
 constexpr size_t kPreMaxImageBytes = size_t(2) << 30;
 
-// Keys from which the magnitudes of a (b, h)'s k and v are worth a launch of
-// their own; below, every workgroup looks through them.
-constexpr int kMaxLaunchKeys = 1024;
+// Keys from which tiles of 128 queries may be split along the keys (the plan's
+// model was fitted there).
+constexpr int kRangeMinKeys = 1024;
 
-// Query tiles of 512 per head from which the presplit pass is used (the
-// break-even of sdpa_bf16.hip's pass, which moves the same bytes).
-template <int kLayout>
-constexpr int kPreMinQueryTiles = kLayout == 1 ? 6 : 12;
+// Query tiles of 512 per head from which the presplit pass is used: the pass
+// against every workgroup splitting the tiles it reads, 8 tiles 424 against 487
+// us (2 x 16 heads, 4096 x 4096) and 116 against 122 (4096 x 1024), 4 tiles 212
+// against 222, key-contiguous k/v 239 against 274 (4 x 16 heads, 2048 x 2048); 2
+// tiles 131 against 130, one 86 against 73.
+constexpr int kPreMinQueryTiles = 4;
 
 template <int kLayout, bool kBias>
 int launch_sized(SdpaParams p, hipStream_t stream) {
@@ -610,55 +743,41 @@ int launch_sized(SdpaParams p, hipStream_t stream) {
   const int64_t ntiles = (p.Lk + kTileKeys - 1) / kTileKeys;
   TilePlan pl;
   if (!plan_tiles(p.B, p.H, p.Lq, p.Lk, wide ? 512 : 128, kTileKeys, kD, wide ? cus : 0, pl)) return kErrDims;
-  const size_t max_bytes = (size_t)heads * kMaxParts * sizeof(uint2);
   // Few queries leave CUs of the 128-query tiles idle: those are split along
-  // the keys, where there is room for the ranges' rows.  (Below kMaxLaunchKeys
-  // every workgroup looks through all of k and v first, whatever its range.)
+  // the keys, where there is room for the ranges' rows.  Elsewhere (a small
+  // caller scratch, no memory, or a capture that would need the workspace to
+  // grow) they run whole, with the sums in one order instead of the ranges'.
   const TilePlan whole = pl;
-  if (!wide && p.Lk >= kMaxLaunchKeys) {
+  if (!wide && p.Lk >= kRangeMinKeys) {
     plan_key_ranges(p.B, p.H, p.Lq, p.Lk, 128, kTileKeys, kD, cus, pl);
-    if (p.scratch != nullptr && pl.scratch_bytes + 256 + max_bytes > p.scratch_bytes) pl = whole;
+    if (p.scratch != nullptr && pl.scratch_bytes > p.scratch_bytes) pl = whole;
   }
   const size_t part_bytes = (pl.scratch_bytes + 255) / 256 * 256;
   const size_t image_bytes = (size_t)heads * ntiles * kImageTileBytes<kBias>;
-  bool image = wide && p.scratch == nullptr && qtiles >= kPreMinQueryTiles<kLayout> &&
+  bool image = wide && p.scratch == nullptr && qtiles >= kPreMinQueryTiles &&
                image_bytes <= kPreMaxImageBytes && heads * ntiles <= 0x7fffffff;
-  uint2* maxes = nullptr;
-  if (p.scratch != nullptr) {
-    // behind the key-split partials, where the caller's scratch has room
-    if (p.Lk >= kMaxLaunchKeys && part_bytes + max_bytes <= p.scratch_bytes)
-      maxes = reinterpret_cast<uint2*>(reinterpret_cast<char*>(p.scratch) + part_bytes);
-  } else if (image || p.Lk >= kMaxLaunchKeys) {
-    // One buffer: partials, magnitudes, image.  Without it (allocation
-    // failure, or a capture that would need it to grow) the workgroups look
-    // through and split k and v themselves, with the same result.
-    void* ws = image ? stream_workspace(stream, part_bytes + max_bytes + image_bytes, kSlotSdpaPartial) : nullptr;
+  uintx4* img = nullptr;
+  if (p.scratch == nullptr && (image || (!wide && pl.pieces > 0))) {
+    // One buffer: partials, image.  Without it the workgroups split k and v
+    // themselves, with the same result.
+    void* ws = stream_workspace(stream, part_bytes + (image ? image_bytes : 0), kSlotSdpaPartial);
     if (ws == nullptr) {
       image = false;
-      if (p.Lk >= kMaxLaunchKeys) ws = stream_workspace(stream, part_bytes + max_bytes, kSlotSdpaPartial);
-    }
-    if (ws == nullptr && !wide) pl = whole;
-    if (ws != nullptr) {
+      if (!wide) pl = whole;
+    } else {
       p.scratch = static_cast<float*>(ws);
       p.scratch_bytes = pl.scratch_bytes;
-      maxes = reinterpret_cast<uint2*>(static_cast<char*>(ws) + part_bytes);
+      img = reinterpret_cast<uintx4*>(static_cast<char*>(ws) + part_bytes);
     }
   }
-  const SdpaArgs a = make_args(p);
-  if (maxes != nullptr) {
-    hipLaunchKernelGGL(sdpa_f16_max_kernel<kLayout>, dim3((unsigned)(heads * kMaxParts)), dim3(kMaxThreads), 0, stream,
-                       a, maxes);
-    if (hipGetLastError() != hipSuccess) return kErrLaunch;
-  }
   if (image) {
-    auto* img = reinterpret_cast<uintx4*>(reinterpret_cast<char*>(maxes) + max_bytes);
     hipLaunchKernelGGL((sdpa_f16_presplit_kernel<kLayout, kBias>), dim3((unsigned)(heads * ntiles)),
-                       dim3(kPreThreads), 0, stream, a, maxes, img, (int)ntiles);
+                       dim3(kPreThreads), 0, stream, make_args(p), img, (int)ntiles);
     if (hipGetLastError() != hipSuccess) return kErrLaunch;
-    return launch_shape<0, kBias, 16, true>(p, stream, pl, maxes, img);
+    return launch_shape<kLayout, kBias, 16, true>(p, stream, pl, img);
   }
-  if (wide) return launch_shape<kLayout, kBias, 16, false>(p, stream, pl, maxes, nullptr);
-  return launch_shape<kLayout, kBias, 4, false>(p, stream, pl, maxes, nullptr);
+  if (wide) return launch_shape<kLayout, kBias, 16, false>(p, stream, pl, nullptr);
+  return launch_shape<kLayout, kBias, 4, false>(p, stream, pl, nullptr);
 }
 
 }  // namespace
