@@ -96,6 +96,7 @@ int sdpa_checked(const float* q, const float* k, const float* v, const float* bi
   if (has_bias) TSPLAT_CHECK(ptrs.check(bias, ((int64_t)(H - 1) * bias_head_stride + Lk) * 4));
   SdpaParams p{q, k, v, has_bias ? bias : nullptr, out, B, H, Lq, Lk, kv_packed, Lkp,
                bias_head_stride, out_blhd, precision, scratch, scratch_bytes};
+  const auto enqueue = hold_enqueue(stream);
   const int st = launch_sdpa(p, stream);
   if (st == kErrLaunch) (void)note(hipErrorLaunchFailure);
   return st;
@@ -131,6 +132,7 @@ int gemm_checked(const float* x, const int16_t* code01, const int8_t* q2, const 
   TSPLAT_CHECK(ptrs.check(bias, (int64_t)N * 4));
   TSPLAT_CHECK(ptrs.check(out, ((int64_t)(M - 1) * stride_out + count) * 4));
   GemmParams p{x, code01, q2, scale, bias, out, M, K, N, start, count, stride_x, stride_out};
+  const auto enqueue = hold_enqueue(stream);
   const int st = launch_nf24_gemm(p, stream);
   if (st == kErrLaunch) (void)note(hipErrorLaunchFailure);
   return st;
@@ -261,6 +263,7 @@ int qkv_direct_checked(const float* x, const int16_t* code01, const int8_t* q2,
                    freqs, qg, kg, q, pk, pv, B, L, H, Lp, fb, kv_layout, kv_round};
   p.gemm.w_hi = with_planes ? w_hi : nullptr;
   p.gemm.w_lo = with_planes && precision == kPrecisionBf16x3 ? w_lo : nullptr;
+  const auto enqueue = hold_enqueue(stream);
   const int st = launch_nf24_gemm_qkv(p, stream);
   if (st == kErrLaunch) (void)note(hipErrorLaunchFailure);
   return st;

@@ -175,6 +175,7 @@ int gemm_precision_checked(const float* x, const int16_t* code01_t, const int8_t
   p.w_hi = w_hi;
   p.w_lo = precision == kPrecisionBf16x3 ? w_lo : nullptr;
   GemmEpilogueParams e{epilogue, gate, gate_stride, rows_per_batch > 0 ? rows_per_batch : 1};
+  const auto enqueue = hold_enqueue(stream);
   return launched(launch_nf24_gemm_epilogue(p, e, stream));
 }
 

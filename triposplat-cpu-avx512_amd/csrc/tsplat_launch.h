@@ -6,6 +6,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <mutex>
+
 namespace tsplat {
 
 // out[m, c] = bias[n0+c] + sum_k x[m, k] * w[k, n0+c],  c in [0, n_count),
@@ -225,6 +227,10 @@ enum WorkspaceSlot : int {
   kSlotSdpaPlanes = 3,  // pre-split bf16 K/V tiles of the bf16 SDPA modes
 };
 void* stream_workspace(hipStream_t stream, size_t bytes, int slot);
+// Held by an entry point over the enqueue of a call that may use a workspace:
+// calls from several host threads on one stream follow one another whole
+// (workspace_pool.h).
+std::unique_lock<std::recursive_mutex> hold_enqueue(hipStream_t stream);
 // Frees the slot's buffers of the current device that no capture recorded
 // (after their streams) and retires the others.
 void release_workspace(int slot);

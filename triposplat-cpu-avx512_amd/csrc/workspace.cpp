@@ -1,8 +1,9 @@
 // Per-stream device workspaces for kernels that need scratch memory: the
 // split-K partial sums of the few-row GEMM, the key-split partials of the
-// SDPA tail and the pre-split K/V tiles of the bf16 SDPA modes.  Every user
-// overwrites the part it reads, so buffers are not cleared.  The grow / free / retire policy is WorkspacePool's
-// (workspace_pool.h); this file supplies the HIP operations and a lock.
+// SDPA tail and the pre-split K/V tiles of the SDPA.  Every user
+// overwrites the part it reads, so buffers are not cleared.  The grow / free /
+// retire policy is WorkspacePool's (workspace_pool.h); this file supplies the
+// HIP operations and the locks.
 
 #include <hip/hip_runtime.h>
 
@@ -55,7 +56,14 @@ Pool& pool() {
   return *g_pool;
 }
 
+EnqueueLocks& enqueue_locks() {
+  static EnqueueLocks* locks = new EnqueueLocks;  // (as the pool: never destroyed)
+  return *locks;
+}
+
 }  // namespace
+
+std::unique_lock<std::recursive_mutex> hold_enqueue(hipStream_t stream) { return enqueue_locks().hold(stream); }
 
 void* stream_workspace(hipStream_t stream, size_t bytes, int slot) {
   int dev = 0;
@@ -78,6 +86,7 @@ void release_workspace(int slot) {
     (void)hipGetLastError();
     return;
   }
+  const auto enqueues = enqueue_locks().hold_all();
   std::lock_guard<std::mutex> lock(g_mu);
   pool().release(dev, slot);
 }

@@ -22,7 +22,10 @@
 //     and buffers of a stream that no longer exists (it cannot be waited
 //     on).  A destroyed stream's buffer is therefore reclaimed only by a
 //     release() made before the stream is destroyed.
-// Calls on one stream are ordered by the stream and share its buffer; a
+// Calls on one stream are ordered by the stream and share its buffer; a call
+// holds its stream's EnqueueLocks entry from before it asks for a buffer until
+// the last launch that uses it is enqueued, so that a call from another host
+// thread neither comes between its launches nor grows the buffer under them.  A
 // graph must be replayed on the stream it was captured on (or ordered with
 // that stream's eager work), since both use the same buffer.  Streams are
 // keyed by handle: a new stream that reuses a destroyed stream's handle
@@ -34,6 +37,7 @@
 #include <stdint.h>
 
 #include <map>
+#include <mutex>
 #include <tuple>
 #include <vector>
 
@@ -157,6 +161,28 @@ class WorkspacePool {
   std::map<std::tuple<int, Stream, int>, WorkspaceBuffer> buffers_;
   std::vector<void*> retired_;
   WorkspaceSlotStats stats_[kSlots];
+};
+
+// One lock per stream (streams are spread over a fixed number of them): held
+// over the enqueue of a call, which may ask for several buffers and call
+// itself for a part of its rows; all of them, in order, by release().
+class EnqueueLocks {
+ public:
+  using Lock = std::unique_lock<std::recursive_mutex>;
+  static constexpr int kLocks = 64;
+  Lock hold(const void* stream) {
+    const uint64_t h = (uint64_t)reinterpret_cast<uintptr_t>(stream) * 0x9e3779b97f4a7c15ull;
+    return Lock(mu_[h >> 58]);
+  }
+  std::vector<Lock> hold_all() {
+    std::vector<Lock> all;
+    for (auto& m : mu_) all.emplace_back(m);
+    return all;
+  }
+
+ private:
+  static_assert(kLocks == 64, "hold() takes six bits");
+  std::recursive_mutex mu_[kLocks];
 };
 
 }  // namespace tsplat
