@@ -4,7 +4,8 @@
 // 256-CU device, the plan must
 //   - run every query tile exactly once: whole, or as key ranges that cover
 //     [0, Lk) once each (ranges a multiple of the key tile, none empty);
-//   - keep all pieces within 2 * CUs - 1;
+//   - keep all pieces within 2 * CUs - 1 (6 * CUs where few tiles are all split,
+//     plan_key_ranges);
 //   - need at most the no-allocation entry point's 66 MiB of scratch;
 //   - refuse a caller scratch one byte smaller than it needs.
 // Built and run by tests/test_sdpa_plan.py; prints "ok <plans checked>" and
@@ -84,6 +85,39 @@ int main() {
               if (pl.scratch_bytes > worst) worst = pl.scratch_bytes;
             }
           }
+  // plan_key_ranges: every tile of a four-wave plan split, or the plan untouched
+  long split = 0;
+  size_t worst_ranges = 0;
+  const int range_lks[] = {1024, 1025, 1087, 1088, 2047, 2048, 2562, 3000, 4100, 8194, 9000, 16384, 16385, 100000};
+  for (long bh = 1; bh <= 600; bh = bh < 40 ? bh + 1 : bh * 3 / 2)
+    for (int Lq = 1; Lq <= 16 * 1024 && bh * ((Lq + 511) / 512) < kCus; Lq = Lq < 520 ? Lq + 37 : Lq * 5 / 4)
+      for (int Lk : range_lks) {
+        TilePlan pl;
+        check(tsplat::sdpa::plan_tiles(1, bh, Lq, Lk, 128, 64, kD, 0, pl), "plan refused", bh, Lq, Lk, 128, 64);
+        tsplat::sdpa::plan_key_ranges(1, bh, Lq, Lk, 128, 64, kD, kCus, pl);
+        ++plans;
+        if (pl.pieces == 0) {
+          check(pl.full_tiles == pl.tiles && pl.scratch_bytes == 0 && pl.grid() == pl.tiles, "ranges: whole", bh, Lq, Lk,
+                128, 64);
+          continue;
+        }
+        ++split;
+        const int64_t partial = Lq % 128 != 0 ? bh : 0;
+        check(pl.full_tiles == 0 && pl.splits >= 2, "ranges: every tile split", bh, Lq, Lk, 128, 64);
+        check(pl.splits == pl.splits_p && pl.keys_per_split == pl.keys_per_split_p, "ranges: one split", bh, Lq, Lk, 128,
+              64);
+        check(ranges_ok(Lk, pl.keys_per_split, pl.splits, 64), "ranges: keys covered once", bh, Lq, Lk, 128, 64);
+        check(pl.pieces == pl.tiles * pl.splits && pl.pieces_full == (pl.tiles - partial) * pl.splits &&
+                  pl.grid() == pl.pieces,
+              "ranges: pieces", bh, Lq, Lk, 128, 64);
+        check(pl.pieces <= 6 * kCus, "ranges: pieces within 6 * CUs", bh, Lq, Lk, 128, 64);
+        check(pl.scratch_bytes == (size_t)pl.pieces * 128 * (kD + 2) * 4 && pl.scratch_bytes <= kNoAllocScratch,
+              "ranges: scratch", bh, Lq, Lk, 128, 64);
+        if (pl.scratch_bytes > worst_ranges) worst_ranges = pl.scratch_bytes;
+      }
+  check(split > 1000, "ranges: plans that split", 0, 0, 0, 0, 0);
+  check(worst_ranges <= (size_t)6 * kCus * 128 * (kD + 2) * 4, "worst split of every tile within the stated bound", 0, 0,
+        0, 0, 0);
   // the bound the comments state: (2 * CUs - 1) pieces of 512 rows x 66 floats
   check(worst <= (size_t)(2 * kCus - 1) * 512 * (kD + 2) * 4, "worst plan within the stated bound", 0, 0, 0,
         0, 0);

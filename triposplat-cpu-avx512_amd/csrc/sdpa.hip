@@ -24,23 +24,21 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_kernel(SdpaArgs a) {
 }
 
 template <int kLayout, bool kBias, int kWaves, int kBKV, bool kSplit>
-int launch_shape(const SdpaParams& p, hipStream_t stream, int cus) {
-  return launch_tiles(make_args(p), p, kWaves * 32, kBKV, cus, stream, [&](dim3 grid, const SdpaArgs& a) {
+int launch_shape(const SdpaParams& p, hipStream_t stream) {
+  return launch_tiles(make_args(p), p, kWaves * 32, kBKV, 0, stream, [&](dim3 grid, const SdpaArgs& a) {
     hipLaunchKernelGGL((sdpa_kernel<kLayout, kBias, kWaves, kBKV, kSplit>), grid, dim3(kWaves * 64), 0,
                        stream, a);
   });
 }
 
-// Grids too small to give every CU one 512-query workgroup use 4 waves;
-// larger grids whose tile count is not a multiple of the CU count split the
-// remainder's keys (launch_tiles).  A key bias runs the per-32-key-block
-// softmax (kSplit).
+// Grids too small to give every CU one 512-query workgroup use 4 waves.  A key
+// bias runs the per-32-key-block softmax (kSplit).  (One key tile: nothing to
+// split along the keys.)
 template <int kLayout, bool kBias>
 int launch_sized(const SdpaParams& p, hipStream_t stream) {
-  const int cus = compute_units();
   const int64_t wide_tiles = (int64_t)p.B * p.H * ((p.Lq + 511) / 512);
-  if (wide_tiles < cus) return launch_shape<kLayout, kBias, 4, 64, false>(p, stream, 0);
-  return launch_shape<kLayout, kBias, 16, 64, kBias>(p, stream, cus);
+  if (wide_tiles < compute_units()) return launch_shape<kLayout, kBias, 4, 64, false>(p, stream);
+  return launch_shape<kLayout, kBias, 16, 64, kBias>(p, stream);
 }
 
 // Fewest keys for the fp16-product kernel (sdpa_f16.hip): one of its key

@@ -9,9 +9,10 @@
 // round fills every CU; each range ("piece") writes its kBQ unnormalised
 // output rows and (max, sum) to scratch, and a merge kernel combines them.
 // Partial query tiles (Lq % kBQ != 0, one per head, numbered after the full
-// tiles) take a split of their own.  Every plan keeps the pieces within
-// 2 * cus - 1, so the scratch a plan needs is at most
-// (2 * cus - 1) * kBQ * (kD + 2) * 4 bytes.
+// tiles) take a split of their own.  Such a plan (plan_tiles) keeps the pieces
+// within 2 * cus - 1, so its scratch is at most (2 * cus - 1) * kBQ * (kD + 2) *
+// 4 bytes; a plan that splits every tile because there are few
+// (plan_key_ranges) keeps them within 6 * cus.
 #pragma once
 
 #include <stddef.h>
