@@ -254,3 +254,15 @@ def test_sampler_backend_reference_name():
 
     assert nsb.NativeSamplerAVX512Backend is nsb.NativeSamplerBackend
     assert nsb.create_triposplat_native_sampler_avx512_backend() == (None, {"enabled": False})
+
+
+def test_abi_version_moves_with_the_bindings():
+    """The bound entry points and their argument lists, per ABI version: a new
+    entry or argument needs a new version (and its line here)."""
+    import zlib
+
+    from tsplat import _lib
+
+    text = ";".join(f"{name}({','.join(a.__name__ for a in args)}){getattr(res, '__name__', res)}"
+                    for name, (args, res) in sorted(_lib.SIGNATURES.items()))
+    assert {5: 40773378}.get(_lib.ABI_VERSION) == zlib.crc32(text.encode()), zlib.crc32(text.encode())

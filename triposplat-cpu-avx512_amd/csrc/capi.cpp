@@ -109,7 +109,7 @@ using namespace tsplat;
 namespace {
 
 constexpr int kHeadDim = 64;
-constexpr int kAbiVersion = 4;
+constexpr int kAbiVersion = 5;
 
 // Profile of the blocking (reference-named) SDPA calls: calls, host time
 // spent growing the key-split workspace (allocate), the rest of the call up

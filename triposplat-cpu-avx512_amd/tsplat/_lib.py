@@ -105,8 +105,8 @@ STATUS_TEXT = {
 # whenever an entry's argument list changes (ABI 3 put kv_round before the
 # stream argument of the asynchronous QKV entries: a library reporting another
 # version would read its arguments shifted) or entries are added (ABI 4: the
-# bf16 weight planes).
-ABI_VERSION = 4
+# bf16 weight planes; ABI 5: the packer's error figures).
+ABI_VERSION = 5
 
 _CACHE: dict[str, ctypes.CDLL] = {}
 
