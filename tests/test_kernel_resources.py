@@ -55,8 +55,21 @@ BUDGET = {
 
 # kernels that must exist (a rename must update this test, not skip it)
 REQUIRED = [
-    ("sdpa", "sdpa_kernelILi0ELb0ELi16ELi64ELb0E"),          # configs[1] headline
-    ("nf24_gemm", "GemmCfgILi256ELi192ELi32ELi4ELi3ELi1ELi0ELb1EEELb1ELi0E"),  # configs[0]
+    ("sdpa_f16", "sdpa_f16_kernelILi0ELb0ELi16ELb1E"),       # strict self attention, L = 16384
+    ("sdpa_f16", "sdpa_f16_kernelILi0ELb1ELi16ELb1E"),       # the same with a key bias
+    ("sdpa_f16", "sdpa_f16_kernelILi1ELb0ELi16ELb1E"),       # key-contiguous k/v
+    ("sdpa_f16", "sdpa_f16_kernelILi0ELb0ELi16ELb0E"),       # without the presplit image (captures, few query tiles)
+    ("sdpa_f16", "sdpa_f16_kernelILi0ELb0ELi4ELb0E"),        # few queries
+    ("sdpa_f16", "sdpa_f16_presplit_kernelILi0ELb0E"),       # the presplit pass
+    ("nf24_gemm_f16", "F16CfgILi256ELi256ELi2ELi4ELi4EEELb1ELi3E"),  # strict gated, 12294 x 4096 x 1024
+    ("nf24_gemm_f16", "F16CfgILi256ELi192ELi4ELi3ELi2EEELb1ELi0E"),  # strict 4096 x 1024 x 3072
+    ("nf24_gemm_f16", "F16CfgILi256ELi192ELi4ELi3ELi2EEELb1ELi1E"),  # strict fused QKV, 8194 rows
+    ("nf24_gemm_f16", "F16CfgILi192ELi256ELi3ELi4ELi2EEELb1ELi2E"),
+    ("nf24_gemm_f16", "F16CfgILi256ELi128ELi8ELi2ELi2EEELb1ELi0E"),
+    ("nf24_gemm_f16", "F16CfgILi128ELi64ELi4ELi1ELi2EEELb1ELi0E"),   # strict small grids
+    ("nf24_gemm_f16", "F16CfgILi128ELi64ELi4ELi1ELi2EEELb0ELi0E"),   # and element-wise loads
+    ("sdpa", "sdpa_kernelILi0ELb0ELi16ELi64ELb0E"),          # fewer than 64 keys
+    ("nf24_gemm", "GemmCfgILi256ELi192ELi32ELi4ELi3ELi1ELi0ELb1EEELb1ELi0E"),  # N % 4 == 2
     ("nf24_gemm", "GemmCfgILi256ELi256ELi32ELi4ELi4ELi1ELi0ELb1EEELb1ELi3E"),  # fused QKV, L = 16384
     ("nf24_gemm", "GemmCfgILi256ELi256ELi16ELi4ELi4ELi1ELi0ELb0EEELb0ELi0E"),  # 256x256 scalar-load path
     ("nf24_gemm", "GemmCfgILi256ELi128ELi32ELi4ELi2ELi1ELi0ELb1EEELb1ELi3E"),  # gated, 8192 x 1024
