@@ -13,13 +13,14 @@ packer.
 roofline: the SDPA kernel's average duration from HIP events on the stream it
 is launched on (torch's current stream), FLOPs per launch as above, against
 the rate three fp16 MFMA products per fp32 product can reach (a third of the
-MI355X's dense 2.5 PFLOP/s; fp32 MFMA peaks at 157.3 TFLOP/s).  traffic: HBM bytes per launch
-from the committed rocprofv3 PMC summary (profiles/), or null.
+MI355X's dense 2.5 PFLOP/s; fp32 MFMA peaks at 157.3 TFLOP/s).  traffic: HBM
+bytes per launch from the committed rocprofv3 PMC summary (profiles/), or null.
 
 cpu_baseline: the reference's own AVX-512 kernel (oracle/_ref, compiled from
 the reference sources) on the host cores, on a bounded sample of the same
 workload (all 16 heads, a subset of query rows against all 16384 keys),
-scaled to TFLOP/s.  Falls back to the oracle port if _ref is absent.
+scaled to TFLOP/s.  Falls back to the oracle port if _ref is absent, on a
+sample of a few seconds.  No host work begins past HOST_BUDGET_S.
 Each timed CPU run follows a device call (alternating order), with all host
 threads and with the reference's published thread counts (SDPA 4, GEMM 8).
 """
@@ -50,13 +51,19 @@ def omp_binding():
     return {k: os.environ.get(k) for k in ("OMP_PROC_BIND", "OMP_PLACES", "OMP_NUM_THREADS")}
 
 METRIC = "NF24 GEMM + exact SDPA TFLOP/s (% MFMA peak) at L=16384; s/denoise step"
-PEAK_FP32_MFMA = 157.3  # TFLOP/s, MI355X dense fp32 matrix
 PEAK_STRICT = 2500.0 / 3.0  # three dense fp16 MFMA products per fp32 product
 PEAK_BF16_MFMA = 2500.0  # TFLOP/s, MI355X dense bf16 matrix
 PEAK_HBM = 8000.0       # GB/s
-# host seconds the configs[4] CPU reference step may take (projected from its
-# first block); beyond it the bench reports the projection instead
-FLOW_CPU_BUDGET_S = 480.0
+# host seconds from the program's start after which no further CPU reference
+# work begins: a whole step that would run past it (projected from its first
+# block) is reported as that projection instead, so that the line is printed
+# within minutes on any host
+HOST_BUDGET_S = 300.0
+START = time.perf_counter()
+
+
+def host_left():
+    return HOST_BUDGET_S - (time.perf_counter() - START)
 
 
 def rope_rmsnorm_host(x, theta=10000.0):
@@ -173,7 +180,7 @@ def cpu_baseline_sdpa(q, k, v, budget_s=12.0, gpu_out=None, gpu_fn=None):
     on a 16-core host: ~1.5 s), else the first `rows` query rows of every
     head against all keys.  Median of 3 after one warmup, with all host
     threads; a second figure uses the reference's published SDPA thread
-    count (4).  With `gpu_out` (the device result, [B, L, H, D]) and the
+    count (4; the oracle port, which takes seconds for 256 rows, has none).  With `gpu_out` (the device result, [B, L, H, D]) and the
     reference build present, the sampled rows of the reference's own output
     are also compared with it (`parity_vs_reference`; the GPU tests' bound
     is 1e-5 * max|v| max-abs).  With `gpu_fn` (one timed device call, ms)
@@ -201,10 +208,12 @@ def cpu_baseline_sdpa(q, k, v, budget_s=12.0, gpu_out=None, gpu_fn=None):
 
     gpu_ms = []
 
+    probe, step = (1024, 128) if kind == "reference" else (64, 64)
+
     def measure(nthreads):
-        run(256, nthreads)  # warmup: K/V pack workspace, page-in, thread pool
-        t1 = run(1024, nthreads)
-        rows = L if t1 * L / 1024 * 3 <= budget_s else max(1024, int(budget_s / 3 / t1 * 1024) // 128 * 128)
+        run(probe // 4, nthreads)  # warmup: K/V pack workspace, page-in, thread pool
+        t1 = run(probe, nthreads)
+        rows = L if t1 * L / probe * 3 <= budget_s else max(probe, int(budget_s / 3 / t1 * probe) // step * step)
         times = []
         for _ in range(3):  # device call, CPU run, alternating
             if gpu_fn is not None:
@@ -219,8 +228,10 @@ def cpu_baseline_sdpa(q, k, v, budget_s=12.0, gpu_out=None, gpu_fn=None):
         parity = parity_stats(got, last[rows], tol_abs=1e-5 * float(np.abs(v).max()))
         parity["rows"] = f"{rows} of {L} query rows, all heads"
     flop = 4.0 * B * H * rows * L * D
-    rows4, t4 = measure(4)
-    flop4 = 4.0 * B * H * rows4 * L * D
+    four = {}
+    if kind == "reference":
+        rows4, t4 = measure(4)
+        four = {"threads4_tflops": 4.0 * B * H * rows4 * L * D / t4 / 1e12, "threads4_seconds_per_call": t4 * L / rows4}
     return {
         "value": flop / t_med / 1e12,
         "unit": "TFLOP/s",
@@ -228,11 +239,11 @@ def cpu_baseline_sdpa(q, k, v, budget_s=12.0, gpu_out=None, gpu_fn=None):
         "host_cpu": host_cpu_model(),
         "host_lscpu": host_cpu_topology(),
         "kind": kind,
-        "sample": f"exact SDPA q8t512 (reference AVX-512 build), B=1 H=16 D=64, {rows} of {L} query rows "
+        "sample": f"exact SDPA q8t512 ({'reference AVX-512 build' if kind == 'reference' else 'oracle port'}), "
+                  f"B=1 H=16 D=64, {rows} of {L} query rows "
                   f"vs all {L} keys; median of 3 = {t_med:.3f} s; {threads} OpenMP threads",
         "seconds_per_call": t_med * L / rows,
-        "threads4_tflops": flop4 / t4 / 1e12,
-        "threads4_seconds_per_call": t4 * L / rows4,
+        **four,
         "order": "device call then CPU run, three times per thread count (median of the CPU runs)",
         "alternating_gpu_ms": gpu_ms,
         "omp": omp_binding(),
@@ -363,7 +374,7 @@ def run_sdpa_variants(torch, dev, host, iters=5, ref_parity=False):
         warm_up(torch, fn)
         ms = sorted(time_events(torch, fn, iters) for _ in range(3))[1]
         tf = flop / (ms * 1e-3) / 1e12
-        res[name] = {"ms": ms, "tflops": tf, "frac_fp32_mfma_peak": tf / PEAK_FP32_MFMA}
+        res[name] = {"ms": ms, "tflops": tf, "frac_strict_mfma_peak": tf / PEAK_STRICT}
         if O is not None:
             fn()
             got = np.ascontiguousarray(out.cpu().numpy().transpose(0, 2, 1, 3))
@@ -463,10 +474,10 @@ def run_gemm(torch, dev, iters, ref_parity=False):
                 cpu_ref[tag + "alternating_gpu_ms"] = gms
             cpu_ref["speedup_gpu_vs_cpu_threads8"] = cpu_ref["threads8_s_per_call"] / (g_ms * 1e-3)
     return {
-        "workload": "configs[0] NF24 Linear X[4096x1024] @ W[1024x3072] + bias, fp32 MFMA accumulate",
+        "workload": "configs[0] NF24 Linear X[4096x1024] @ W[1024x3072] + bias, strict products",
         "ms": g_ms,
         "tflops": g_tf,
-        "frac_fp32_mfma_peak": g_tf / PEAK_FP32_MFMA,
+        "frac_strict_mfma_peak": g_tf / PEAK_STRICT,
         "algorithmic_bytes": float(M * K * 4 + K * N * 3 + N * 8 + M * N * 4),
         "traffic": load_traffic("nf24_gemm_config0"),
         "opt_in_bf16": opt_in,
@@ -504,7 +515,7 @@ GEMM_L16384 = (("qkv", 1024, 3072), ("mlp_fc1", 1024, 4096), ("mlp_fc2", 4096, 1
 
 def run_gemm_l16384(torch, dev, iters=8):
     """The flow block's four NF24 Linear shapes at the metric's L = 16384 rows
-    (strict fp32 MFMA, plain store), TFLOP/s and fraction of the fp32 peak."""
+    (strict products, plain store), TFLOP/s and fraction of the strict peak."""
     import numpy as np
     from tsplat.nf24 import nf24_linear
 
@@ -520,7 +531,7 @@ def run_gemm_l16384(torch, dev, iters=8):
     ms = time_interleaved(torch, fns, iters)
     for name, (K, N) in meta.items():
         tf = 2.0 * M * N * K / (ms[name] * 1e-3) / 1e12
-        res[name] = {"M": M, "K": K, "N": N, "ms": ms[name], "tflops": tf, "frac_fp32_mfma_peak": tf / PEAK_FP32_MFMA}
+        res[name] = {"M": M, "K": K, "N": N, "ms": ms[name], "tflops": tf, "frac_strict_mfma_peak": tf / PEAK_STRICT}
     return res
 
 
@@ -582,7 +593,7 @@ def run_reference_shapes(torch, dev, with_cpu, iters=5):
         ms = time_interleaved(torch, {"x": fn}, iters)["x"]
         flop = 4.0 * H * Lq * Lk * D
         row = {"Lq": Lq, "Lk": Lk, "key_bias": "log(4101) on key Lk-1" if logm else None, "ms": ms,
-               "tflops": flop / (ms * 1e-3) / 1e12, "frac_fp32_mfma_peak": flop / (ms * 1e-3) / 1e12 / PEAK_FP32_MFMA}
+               "tflops": flop / (ms * 1e-3) / 1e12, "frac_strict_mfma_peak": flop / (ms * 1e-3) / 1e12 / PEAK_STRICT}
         if name in PUBLISHED_S:
             row["published_cpu_s_4cpu_gcc9_gcc13"] = PUBLISHED_S[name]
             row["speedup_vs_published_gcc13"] = PUBLISHED_S[name][1] / (ms * 1e-3)
@@ -615,7 +626,7 @@ def run_reference_shapes(torch, dev, with_cpu, iters=5):
         ms = time_interleaved(torch, {"x": fn}, iters)["x"]
         flop = 2.0 * M * N * K
         row = {"M": M, "K": K, "N": N, "ms": ms, "tflops": flop / (ms * 1e-3) / 1e12,
-               "frac_fp32_mfma_peak": flop / (ms * 1e-3) / 1e12 / PEAK_FP32_MFMA,
+               "frac_strict_mfma_peak": flop / (ms * 1e-3) / 1e12 / PEAK_STRICT,
                "published_cpu_s_4cpu_gcc9_gcc13": PUBLISHED_S[name],
                "speedup_vs_published_gcc13": PUBLISHED_S[name][1] / (ms * 1e-3)}
         if O is not None:
@@ -718,7 +729,8 @@ def run_flow(torch, dev, steps, with_cpu, validate):
     }
     if with_cpu or validate:
         out["config4_step"]["cpu_reference_full_step"] = flow_step_vs_cpu(
-            torch, dev, model, cfg, z_h, c_h, zn, v, step_s, out["config3_block"])
+            torch, dev, model, cfg, z_h, c_h, zn, v, step_s, out["config3_block"],
+            forced=validate)
     del model
     out["joint"] = run_flow_joint(torch, dev, steps, with_cpu)
     return out
@@ -728,7 +740,7 @@ class _CpuBudget(Exception):
     pass
 
 
-def flow_step_vs_cpu(torch, dev, model, cfg, z_h, c_h, zn, v, step_s, block_row):
+def flow_step_vs_cpu(torch, dev, model, cfg, z_h, c_h, zn, v, step_s, block_row, forced=False):
     """configs[4]'s whole step on the host through the reference's own AVX-512
     kernels (oracle/_ref; the oracle port when that is absent): all 28 blocks
     on both CFG branches, the final layer, CFG and the Euler update, from the
@@ -737,10 +749,11 @@ def flow_step_vs_cpu(torch, dev, model, cfg, z_h, c_h, zn, v, step_s, block_row)
     schedule (dt = 1/58) and of the one-step s1 schedule (dt = 1), each with
     the statistics of scripts/compare_latent_npz.py:22-48 reduced to RMSE,
     max-abs, p99 and the NaN / Inf count; gates: latent RMSE <= 1e-4 and no
-    NaN / Inf.  configs[3]'s block parity comes from the same run: the hidden
-    state after block 0 on both sides.  The host step is abandoned (and only
-    estimated from its first block) if that block projects it past
-    FLOW_CPU_BUDGET_S."""
+    NaN / Inf.  Without the reference's build the step runs only when `forced`
+    (the port takes minutes for a block).  configs[3]'s block parity comes from the same run: the hidden
+    state after block 0 on both sides.  Unless forced, the host step is
+    abandoned (and only estimated from its first block) if that block projects
+    it past the host's budget."""
     import numpy as np
 
     sys.path.insert(0, str(ROOT / "oracle"))
@@ -748,6 +761,8 @@ def flow_step_vs_cpu(torch, dev, model, cfg, z_h, c_h, zn, v, step_s, block_row)
     from flow_ref import CpuFlow, latent_stats, non_finite
 
     backend = "reference" if O.ref_available() else "oracle"
+    if not forced and (backend == "oracle" or host_left() <= 0.0):
+        return None
     dev_after0 = {}
     model.euler_cfg_step(torch.from_numpy(z_h).to(dev), torch.from_numpy(c_h).to(dev), step=0,
                          observe=lambda i, x: dev_after0.setdefault(i, x.cpu().numpy()) if i == 1 else None)
@@ -762,7 +777,7 @@ def flow_step_vs_cpu(torch, dev, model, cfg, z_h, c_h, zn, v, step_s, block_row)
 
     def progress(i):
         el = time.perf_counter() - t0
-        if i == 0 and el * cfg.blocks > FLOW_CPU_BUDGET_S:
+        if i == 0 and not forced and el * (cfg.blocks - 1) > host_left():
             raise _CpuBudget(el)
         if (i + 1) % 7 == 0:
             print(f"cpu configs[4] step: block {i + 1}/{cfg.blocks} ({el:.0f} s)", file=sys.stderr, flush=True)
@@ -896,21 +911,36 @@ def run_flow_joint_reference_shapes(torch, dev, steps, with_cpu=False):
     zn3, _, cn3, _ = model.euler_cfg_step(z, c, cam, reduce_work=True)
     zn3, cn3 = zn3.cpu().numpy(), cn3.cpu().numpy()
     model.set_precision("fp32")
-    cpu_res = None
+    cpu_res = zc = None
     if with_cpu:
         sys.path.insert(0, str(ROOT / "oracle"))
         import numpy as np
         import oracle as O
         from flow_ref import CpuJointFlow, combined_rmse, combined_rmse_from_key_mse, latent_stats, non_finite
 
-        if O.ref_available():
+        if O.ref_available() and host_left() > 0.0:
             cpu = CpuJointFlow(model.host(), cfg, backend="reference", threads=HOST_THREADS)
             t0 = time.perf_counter()
-            cpu.progress = lambda i: (print(f"cpu joint step: block {i + 1}/{cfg.blocks} "
-                                            f"({time.perf_counter() - t0:.0f} s)", file=sys.stderr, flush=True)
-                                      if (i + 1) % 7 == 0 else None)
-            zc, vc, cc, vcc = cpu.joint_euler_cfg_step(z_h, c_h, camera_state(cfg, SEEDS["flow_camera"]))
+
+            done = []
+
+            def progress(i):  # (one branch after the other, each over all blocks)
+                el = time.perf_counter() - t0
+                done.append(i)
+                if len(done) == 1 and el * (2 * cfg.blocks - 1) > host_left():
+                    raise _CpuBudget(el)
+                if (i + 1) % 7 == 0:
+                    print(f"cpu joint step: block {i + 1}/{cfg.blocks} ({el:.0f} s)", file=sys.stderr, flush=True)
+
+            cpu.progress = progress
+            try:
+                zc, vc, cc, vcc = cpu.joint_euler_cfg_step(z_h, c_h, camera_state(cfg, SEEDS["flow_camera"]))
+            except _CpuBudget as e:
+                zc = None
+                cpu_res = {"kind": "reference", "cores": HOST_THREADS,
+                           "s_per_denoise_step_estimated": float(e.args[0]) * 2 * cfg.blocks}
             cpu_s = time.perf_counter() - t0
+        if O.ref_available() and cpu_res is None and zc is not None:
             keys = {"latent": latent_stats(zc, zn), "camera": latent_stats(cc, cn)}
             rel = lambda ref, got: combined_rmse(got, ref) / float(np.sqrt(np.mean(ref.astype(np.float64) ** 2)))
             cpu_res = {
