@@ -242,3 +242,18 @@ def test_tokens_of_any_size(cuda, Lq):
         r = np.nonzero(want[:64] == i)[0]
         # scores of about 375, fp32's last place of which is 2^-16
         assert stats(got[:, :, r] / size[i], exact[:, :, r] / size[i])["rel_rmse"] < 1e-4, i
+
+
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("Lq", [40, 8200])
+def test_masked_first_block_of_few_keys(cuda, Lq, packed):
+    """Fewer keys than a key tile (the fp32 tiles), the first 32 of them masked
+    by -inf: the block adds nothing, and the others are the result."""
+    import torch
+
+    H, Lk = (2, 50) if Lq < 100 else (16, 50)
+    q, k, v = _qkv(31, 1, H, Lq, Lk)
+    b = np.zeros(Lk, np.float32)
+    b[:34] = -np.inf
+    got = _run(torch, cuda, q, k, v, b, packed=packed)[:, :, :64]
+    assert stats(got, sdpa_f64(q[:, :, :64], k[:, :, 34:], v[:, :, 34:]))["rel_rmse"] < 2e-6
