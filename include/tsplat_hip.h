@@ -318,7 +318,9 @@ int tsplat_nf24_gemm_epilogue_async(const float* x, const int16_t* code01_t, con
 /* No counterpart in the reference, whose NF24 Linear is fp32 only; its
  * bf16 evidence is a round-trip probe (triposplat_bf16_roundtrip_patch.py:
  * 7-53, torch's round-to-nearest-even float32 -> bfloat16).  `precision`:
- *   0 strict: fp32 products (the result of tsplat_nf24_gemm_epilogue_async)
+ *   0 strict: products of the fp32 values, carried as fp16 pairs where those
+ *             hold them to fp32's precision and else as they are (the result
+ *             of tsplat_nf24_gemm_epilogue_async)
  *   1 bf16:   bf16(x) * bf16(w) on bf16 MFMA, fp32 accumulation
  *   2 bf16x3: xh*wh + xh*wl + xl*wh, xh = bf16(x), xl = bf16(x - xh), same
  *             for w; about 16 significant bits per product

@@ -9,9 +9,9 @@
 // the reference's sequential fmaf chain.
 //
 // Of the strict calls of more than 32 rows the fp16-product kernel
-// (nf24_gemm_f16.hip, 2.1-2.7x faster) takes all that its loads allow
-// (gemm_f16_takes); the tiles here serve the others, from 256 rows and
-// columns on.
+// (nf24_gemm_f16.hip, 1.7-2.6x faster) takes those that gemm_f16_takes states;
+// the tiles here serve the others: operands that only their two-column or
+// element-wise loads take.
 //
 // Tiling: a workgroup computes a BM x BN output tile with WM x WN waves; a
 // wave owns (BM/WM) x (BN/WN) = MB x NB blocks of 32x32.  Per K step of BK,

@@ -327,9 +327,10 @@ int launch_gemm_f16(const GemmParams& p, int epi, const QkvArgs& e, const GemmEp
 // bf16-mode call, on the strict few-row path (nf24_gemm.hip) with epilogue
 // kind epi: as whole calls of at most 32 rows in every mode, the weight
 // stream is the cost there and fp32 is free.
-int fp32_tail_rows(int M, int n_count);  // how many rows nf24_gemm.hip's tiles split off
 int launch_strict_tail(const GemmParams& p, int epi, const QkvArgs& e, const GemmEpilogueParams& ep,
                        int row0, hipStream_t stream);
+// How many rows nf24_gemm.hip's tiles split off a call as such a tail.
+int fp32_tail_rows(int M, int n_count);
 
 }  // namespace nf24
 }  // namespace tsplat

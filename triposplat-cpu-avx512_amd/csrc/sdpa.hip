@@ -1,6 +1,7 @@
-// Exact online-softmax SDPA for gfx950 (head dim 64, fp32 throughout).  Calls
-// of at least kF16MinKeys keys run on the fp16 matrix cores instead
-// (sdpa_f16.hip, 1.3-2.9x faster).
+// Exact online-softmax SDPA for gfx950 (head dim 64) on fp32 MFMA.  Serves the
+// strict calls of fewer than kF16MinKeys keys; the others run on the fp16
+// matrix cores (sdpa_f16.hip, 1.2-2.8x faster), whose workgroups take the same
+// tile for keys that fp16 pairs do not hold.
 //
 // Reference semantics: scripts/native_sdpa_avx512_exact_q8t512.c:137-332 and
 // the packed/BLHD variant scripts/native_sdpa_avx512_exact_q8t512_packed.c:3-158:
@@ -42,8 +43,8 @@ int launch_sized(const SdpaParams& p, hipStream_t stream) {
 }
 
 // Fewest keys for the fp16-product kernel (sdpa_f16.hip): one of its key
-// tiles.  16 heads of 12294 queries over 65 keys take it 88 us, the kernel
-// here 115; below a tile both are bound by the launch and the queries' loads,
+// tiles.  16 heads of 12294 queries over 65 keys take it 89 us, the kernel
+// here 109; below a tile both are bound by the launch and the queries' loads,
 // and a single key's value comes back exactly here.
 constexpr int kF16MinKeys = 64;
 

@@ -14,7 +14,8 @@ namespace tsplat {
 // w[k, n] = fp32((int32)code01[k, n] * 256 + q2[k, n]) * scale[n].
 //
 // Product precision (opt-in; kPrecisionFp32 is the strict default):
-//   kPrecisionFp32:   fp32 x * fp32 w on fp32 MFMA.
+//   kPrecisionFp32:   fp32 x * fp32 w: three fp16 products per fp32 product
+//                     (nf24_gemm_f16.hip) or fp32 MFMA (nf24_gemm.hip).
 //   kPrecisionBf16:   bf16(x) * bf16(w) on bf16 MFMA, fp32 accumulation;
 //                     bf16() rounds to nearest even from the fp32 value.
 //   kPrecisionBf16x3: x = xh + xl, w = wh + wl with xh = bf16(x),
@@ -61,13 +62,14 @@ struct SdpaParams {
   int Lkp;             // key stride of the packed layout
   int64_t bias_head_stride;  // 0: one [Lk] row shared by all heads
   int out_blhd;        // 1: write [B, Lq, H, 64]
-  // Product precision of Q K^T and P V (GemmPrecision): kPrecisionFp32 on
-  // fp32 MFMA (default); kPrecisionBf16 / kPrecisionBf16x3 split the
+  // Product precision of Q K^T and P V (GemmPrecision): kPrecisionFp32
+  // (default) three fp16 products per fp32 product (sdpa_f16.hip) or fp32
+  // MFMA (sdpa.hip); kPrecisionBf16 / kPrecisionBf16x3 split the
   // operands into bf16 terms as the NF24 GEMM's modes do (q scaled first,
   // p = the unnormalised exponentials); softmax arithmetic stays fp32.
   int precision = kPrecisionFp32;
-  // Scratch for the key-split partials of a partial last round of query
-  // tiles: null takes the stream's library-owned workspace (which may
+  // Scratch for the key-split partials (of a partial last round of query
+  // tiles, or of a whole strict call of few queries): null takes the stream's library-owned workspace (which may
   // allocate); non-null uses [scratch, scratch + scratch_bytes) and fails
   // with kErrScratch when the launch plan needs more.
   float* scratch = nullptr;
@@ -222,7 +224,7 @@ int launch_nf24_decode(const int16_t* code01_t, const int8_t* q2_t, const float*
 // the stream, retire a buffer a capture recorded) is in workspace_pool.h.
 enum WorkspaceSlot : int {
   kSlotGemvPartial = 0,
-  kSlotSdpaPartial = 1,
+  kSlotSdpaPartial = 1,  // key-split partials and the strict SDPA's K/V image
   kSlotGemmTail = 2,
   kSlotSdpaPlanes = 3,  // pre-split bf16 K/V tiles of the bf16 SDPA modes
 };
