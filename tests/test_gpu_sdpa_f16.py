@@ -257,3 +257,22 @@ def test_masked_first_block_of_few_keys(cuda, Lq, packed):
     b[:34] = -np.inf
     got = _run(torch, cuda, q, k, v, b, packed=packed)[:, :, :64]
     assert stats(got, sdpa_f64(q[:, :, :64], k[:, :, 34:], v[:, :, 34:]))["rel_rmse"] < 2e-6
+
+
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("H,Lq,Lk", [(2, 70, 300), (2, 70, 1200), (16, 8200, 300)])
+@pytest.mark.parametrize("mask", [-1e9, -1e30])
+@pytest.mark.parametrize("level", [-30.0, -60.0])
+def test_first_keys_under_a_finite_mask(cuda, H, Lq, Lk, mask, level, packed):
+    """The reference starts at a mask of many digits and then has to be the live
+    keys', however low they lie.  (Scores of up to 100 log2 units are held to 2^-18:
+    2.6e-6 of a weight, beside the 2e-6 of the other cases.)"""
+    import torch
+
+    q, k, v = _qkv(int(-level) + Lk, 1, H, Lq, Lk)
+    print(f"sdpa first keys masked H={H} Lq={Lq} Lk={Lk} mask={mask} level={level} packed={packed}", flush=True)
+    b = np.full(Lk, level, np.float32)
+    b[:70] = mask
+    got = _run(torch, cuda, q, k, v, b, packed=packed)[:, :, :64]
+    exact = sdpa_f64(q[:, :, :64], k[:, :, 70:], v[:, :, 70:])
+    assert stats(got, exact)["rel_rmse"] < 4.6e-6

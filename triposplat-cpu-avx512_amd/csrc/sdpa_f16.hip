@@ -620,10 +620,6 @@ void sdpa_f16_kernel(SdpaArgs a, const uintx4* pre) {
 #pragma unroll
               for (int e = 0; e < 4; ++e) s[4 * r4 + e] = fmaf(s[4 * r4 + e], c1, bb[e] - sub);
             }
-            if (huge) {
-#pragma unroll
-              for (int r = 0; r < 16; ++r) s[r] = (s[r] - m_ref) + kPBase;
-            }
           }
           if (tail) {
             const int valid = a.Lk - key0 - 4 * g;
@@ -635,7 +631,16 @@ void sdpa_f16_kernel(SdpaArgs a, const uintx4* pre) {
 #pragma unroll
           for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[r]);
           mx = pair_max(mx);
-          mx = kBias ? (mx - kPBase) + m_ref : mx * c1;
+          if constexpr (!kBias) {
+            mx *= c1;
+          } else if (huge) {
+            // (the maximum from the scores as they are: the next reference has
+            // to be exact also where this one is a mask of many digits)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s[r] = (s[r] - m_ref) + kPBase;
+          } else {
+            mx = (mx - kPBase) + m_ref;
+          }
           const bool move = fresh ? mx > -INFINITY : mx > m_run + kSlack;
           if (__builtin_amdgcn_ballot_w64(move) == 0) break;
           const float m_new = move ? mx : m_run;
