@@ -276,3 +276,22 @@ def test_first_keys_under_a_finite_mask(cuda, H, Lq, Lk, mask, level, packed):
     got = _run(torch, cuda, q, k, v, b, packed=packed)[:, :, :64]
     exact = sdpa_f64(q[:, :, :64], k[:, :, 70:], v[:, :, 70:])
     assert stats(got, exact)["rel_rmse"] < 4.6e-6
+
+
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("H,Lq,Lk,masked", [(2, 70, 300, 0), (2, 70, 300, 70), (2, 70, 1200, 1030),
+                                            (16, 8200, 300, 0), (16, 8200, 300, 70)])
+@pytest.mark.parametrize("log2_level", [-2.9e38, -3.0e38, -3.3e38])
+def test_bias_at_the_end_of_the_range(cuda, H, Lq, Lk, masked, log2_level, packed):
+    """A bias that leaves every live key the same score near fp32's lowest: all of
+    them weigh the same, in one part or merged with parts that are masked whole."""
+    import torch
+
+    level = np.float32(log2_level / math.log2(math.e))
+    print(f"sdpa bias {level} H={H} Lq={Lq} Lk={Lk} masked={masked} packed={packed}", flush=True)
+    q, k, v = _qkv(masked + Lk, 1, H, Lq, Lk)
+    b = np.full(Lk, level, np.float32)
+    b[:masked] = -np.inf
+    got = _run(torch, cuda, q, k, v, b, packed=packed)[:, :, :64]
+    exact = np.broadcast_to(v[:, :, masked:].astype(np.float64).mean(axis=2, keepdims=True), got.shape)
+    assert np.abs(got - exact).max() <= 2.0 ** -20 * np.abs(v).max()

@@ -83,7 +83,9 @@ constexpr int kWaitVmcnt0 = 0x0f70;  // s_waitcnt operand: vector-memory count 0
 // score's own.
 constexpr float kPBase = 4.0f;
 constexpr float kSlack = 4.0f;
-constexpr float kStart = -3.0e38f;   // the reference before any key
+// The reference before any key: no key's own, which ends the search for it (a
+// bias may make a finite score of any size).
+constexpr float kStart = -INFINITY;
 // Largest |q| |k| (of a wave's queries, of a key tile) whose scores the pairs
 // serve: any, short of the scales' own range, where neither operand's values
 // spread over more than its pairs hold; elsewhere as long as 64 dims of 2^-39
@@ -644,7 +646,7 @@ void sdpa_f16_kernel(SdpaArgs a, const uintx4* pre) {
           const bool move = fresh ? mx > -INFINITY : mx > m_run + kSlack;
           if (__builtin_amdgcn_ballot_w64(move) == 0) break;
           const float m_new = move ? mx : m_run;
-          const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+          const float alpha = move ? __builtin_amdgcn_exp2f(m_run - m_new) : 1.0f;
           l_run *= alpha;
 #pragma unroll
           for (int db = 0; db < 2; ++db)
@@ -710,7 +712,8 @@ void sdpa_f16_kernel(SdpaArgs a, const uintx4* pre) {
     for (int db = 0; db < 2; ++db)
 #pragma unroll
       for (int r = 0; r < 16; ++r) o[db][r] = __builtin_amdgcn_ldexpf(o[db][r], -(int)kPBase - kPShift - ev);
-    store_rows<kBQ>(e, o, m_run, l_run * 0x1p-11f, tid_e);
+    // (without a key, the fp32 tiles' reference, which is no larger than a key's)
+    store_rows<kBQ>(e, o, fmaxf(m_run, -FLT_MAX), l_run * 0x1p-11f, tid_e);
     if (v_inf == 0) return;
   }
   __syncthreads();
