@@ -295,3 +295,21 @@ def test_bias_at_the_end_of_the_range(cuda, H, Lq, Lk, masked, log2_level, packe
     got = _run(torch, cuda, q, k, v, b, packed=packed)[:, :, :64]
     exact = np.broadcast_to(v[:, :, masked:].astype(np.float64).mean(axis=2, keepdims=True), got.shape)
     assert np.abs(got - exact).max() <= 2.0 ** -20 * np.abs(v).max()
+
+
+@pytest.mark.parametrize("Lq,Lk", [(70, 300), (70, 1200), (8200, 300)])
+def test_scores_that_a_bias_takes_back(cuda, Lq, Lk):
+    """Scores and a bias of 2^30 each, one above the other by a few hundred log2
+    units: equal keys keep equal weights."""
+    import torch
+
+    H = 2 if Lq < 100 else 16
+    q, k, v = _qkv(3, 1, H, Lq, Lk)
+    print(f"sdpa bias takes scores back Lq={Lq} Lk={Lk}", flush=True)
+    q[:], k[:] = 0.0, 0.0
+    q[..., 0] = np.float32(2.0 ** 15)
+    k[..., 0] = np.float32(2.0 ** 18 * (1 + 2.0 ** -22))
+    b = np.full(Lk, -(2.0 ** 30), np.float32)
+    got = _run(torch, cuda, q, k, v, b)[:, :, :64]
+    exact = np.broadcast_to(v.astype(np.float64).mean(axis=2, keepdims=True), got.shape)
+    assert np.abs(got - exact).max() <= 2.0 ** -20 * np.abs(v).max()

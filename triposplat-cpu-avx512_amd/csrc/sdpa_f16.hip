@@ -96,6 +96,8 @@ constexpr int kEvRange = 1024;  // beyond any ev
 // of one tile stay in range in that of another.
 constexpr int kEvSpread = 64;
 constexpr float kWideTop = 0x1p14f;
+// |q| |k| from which 64 dims may score 2^20 log2 units (2^19.5 here).
+constexpr float kFarScores = 0x1p16f;
 // p is taken up by 2^kPShift before it is split: below 2^15, and held to 2^-25,
 // 2^-36 of a weight at the reference (many small weights add up: 16384 of them,
 // each 2^-30 of one key's, were lost to the pairs, not to their sum).  After the
@@ -520,8 +522,9 @@ void sdpa_f16_kernel(SdpaArgs a, const uintx4* pre) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) o[db][r] = 0.0f;
   float m_run = kStart;  // the reference
-  // some query's reference is beyond 2^20 (uniform over the wave): exponents
-  // are then differences of rounded scores, 0 at the maximum
+  // some query's reference, or with a bias a score before it, may be beyond 2^20
+  // (uniform over the wave): exponents are then differences of rounded scores, 0
+  // at the maximum
   bool huge = false;
   float l_run = 0.0f;
   int ev = 0;  // the outputs' unit: 2^-ev
@@ -580,6 +583,7 @@ void sdpa_f16_kernel(SdpaArgs a, const uintx4* pre) {
       // so that a masked score stays -inf
       const float c1 =
           __builtin_amdgcn_fmed3f(__builtin_amdgcn_ldexpf(0.125f * kLog2e, -eq - info.ek), 0x1p-126f, 0x1p127f);
+      if (kBias) huge |= qmax * info.kmax > kFarScores;
       if (info.ev != ev && (info.flags & kVZero) == 0) {
 #pragma unroll
         for (int db = 0; db < 2; ++db)
