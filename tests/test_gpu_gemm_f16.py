@@ -165,6 +165,27 @@ def test_large_values_without_weight(oracle, cuda, hiplib, M, N, dead):
     assert np.array_equal(got[keep].view(np.uint32), plain[keep].view(np.uint32))
 
 
+@pytest.mark.parametrize("M,N", [(40, 64), (300, 1028)])
+@pytest.mark.parametrize("dead", [[5], [40]])
+def test_values_that_the_row_scale_takes_to_zero(oracle, cuda, hiplib, M, N, dead):
+    """A value times its row's scale may be zero in fp32 and still be all that the
+    results consist of."""
+    import torch
+
+    x, c01, q2, s, b = _dead_features(oracle, M + N, M, 160, N, dead)
+    b[:] = 0.0
+    print(f"gemm f16 to zero M={M} N={N} dead={dead}", flush=True)
+    y = x.copy()
+    rows = {1: (1e30, 1e-18), 8: (3e38, 1e-9), 33: (-3e38, 1e-25)}
+    for r, (large, f) in rows.items():
+        y[r] *= np.float32(f)
+        y[r, dead] = large
+    got = _run(torch, y, c01, q2, s, b)
+    w = oracle.decode_nf24(c01, q2, s)
+    pick = list(rows)
+    assert np.all(np.abs(got[pick] - gemm_f64(y[pick], w, b)) <= gemm_order_bound(y[pick], w, b))
+
+
 @pytest.mark.parametrize("M,N", [(40, 64), (300, 1024)])
 def test_ends_of_the_range(oracle, cuda, hiplib, M, N):
     """Finite results of huge and tiny rows (the decoded weights are small) stay finite and exact."""

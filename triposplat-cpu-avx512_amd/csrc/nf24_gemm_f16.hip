@@ -43,7 +43,7 @@
 // A call pays for such rows with the second pass: 4096 x 1024 x 3072 with one
 // value of 1e6 80 -> 180 us (fp32 tiles: 196), a feature 3000 times the others
 // 213, 1e5 times 262; 600 times, in the first pass, 90 (with a headroom of 2^9
-// and without the shift of xl: 197).
+// and without the shift of xl: 197); all of x times 1e10 (a scan, kSmallScale) 141.
 //
 // Tiling: BM x BN workgroup tile, WM x WN waves, a wave owns MB x NB blocks
 // of 32 x 32 (the accumulator layout the epilogues of nf24_gemm_common.h
@@ -100,6 +100,7 @@ struct F16Cfg {
   static_assert(WK == 2 || WK == 4, "W units are 2 or 4 k rows deep");
   static_assert(kXUnits % 64 == 0 && kWUnits % 64 == 0, "a partial iteration must cover whole waves");
   static_assert(kTM % 32 == 0 && kTN % 32 == 0, "wave tile must be 32-aligned");
+  static_assert(kThreads >= BM, "a thread for every row");
   // unit j of this thread exists (uniform over a wave)
   template <int kUnits, int kIter>
   __device__ static constexpr bool unit(int tid, int j) {
@@ -155,6 +156,11 @@ __device__ __forceinline__ void store_pairs(_Float16* dst, const unsigned (&w)[N
 // reaches kUnitMin.
 constexpr float kRowTop = 65520.0f;
 constexpr uint32_t kUnitMin = (127u - 17u) << 23;  // bits of 2^-17
+// Scales that may take a normal value to zero (a unit of those looks like zeros
+// while it is staged): rows under one are looked at again, and their pairs serve
+// where that befalls no value.  (A check of x instead of x * s while staging: 600 x
+// 1024 x 1024 28.7 against 26.5 us.)
+constexpr float kSmallScale = 0x1p-23f;
 
 // The power of two that brings a magnitude (as bits) to [2^kTop, 2^(kTop + 1)),
 // with a normal reciprocal.
@@ -429,7 +435,7 @@ void nf24_gemm_f16_kernel(GemmArgs a) {
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             const float w = k + u * C::BK + e < a.K ? fabsf(v[u][e] * s) : 0.0f;
-            bad |= !(w < kRowTop);
+            bad |= !(w < kRowTop) || (s < kSmallScale && w == 0.0f && v[u][e] != 0.0f);
             mx = max(mx, __float_as_uint(w));
           }
           bad |= mx - 1u < kUnitMin - 1u;
@@ -570,12 +576,15 @@ void nf24_gemm_f16_kernel(GemmArgs a) {
       for (int nb = 0; nb < C::kNB; ++nb)
 #pragma unroll
         for (int r = 0; r < 16; ++r) chk = fmaf(acc[mb][nb][r], 0.0f, chk);
-    if (!__builtin_amdgcn_readfirstlane(__syncthreads_or(chk != 0.0f || low < kUnitMin - 1u))) break;
-    rest = __builtin_amdgcn_readfirstlane(second) != 0;
     asm volatile("" : "+v"(tid_x));
+    const bool bad = chk != 0.0f || low < kUnitMin - 1u || row_sc[min(tid_x, C::BM - 1)] < kSmallScale;
+    if (!__builtin_amdgcn_readfirstlane(__syncthreads_or(bad))) break;
+    rest = __builtin_amdgcn_readfirstlane(second) != 0;
     find_rows(tid_x);
     __syncthreads();
-    if (rest) break;
+    const bool any = __builtin_amdgcn_readfirstlane(__syncthreads_or(row_flag[min(tid_x, C::BM - 1)])) != 0;
+    rest = rest && any;
+    if (rest || !any) break;
     // Those rows' scales from the whole row, and once more (the other rows' sums
     // come out as they were).
     if (tid == 0) second = 1;
