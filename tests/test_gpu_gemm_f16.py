@@ -6,9 +6,9 @@ NaNs, and codes over the format's whole range.
 Bound.  Each operand is carried as two fp16 values that hold it to one unit of
 fp32's last place, the dropped product of the low parts is below 2^-22 of the
 term, and the sums are fp32: within _parity.gemm_order_bound for K >= 64.  A
-value of x below 2^-24 of its row's scale is rounded to 2^-25 of the scale,
-2^-31 of the largest of the values the scale was set from (the row's first 32,
-or all of them when those are zero): 2^-31 * max|x_row| * sum_k |w_k| covers it.
+value of x is held to 2^-36 in the unit in which the largest of the values the
+scale was set from (the row's first 32, or all of them when those are zero or the
+row is taken again) is at least 2^3: 2^-39 * max|x_row| * sum_k |w_k| covers it.
 """
 from __future__ import annotations
 
@@ -29,7 +29,7 @@ def _run(torch, x, c01, q2, s, b):
 
 def _check(oracle, x, c01, q2, s, b, got):
     w = oracle.decode_nf24(c01, q2, s)
-    floor = 2.0 ** -31 * np.abs(x.astype(np.float64)).max(1)[:, None] * np.abs(w.astype(np.float64)).sum(0)[None]
+    floor = 2.0 ** -39 * np.abs(x.astype(np.float64)).max(1)[:, None] * np.abs(w.astype(np.float64)).sum(0)[None]
     exact = gemm_f64(x, w, b)
     assert np.all(np.isfinite(got))
     assert np.all(np.abs(got - exact) <= gemm_order_bound(x, w, b) + floor), float(np.abs(got - exact).max())
